@@ -106,7 +106,8 @@ EXPORTS = (
     "adambridge_pool_sync", "adambridge_set_stream", "adambridge_last_error", "adambridge_backend",
     "adambridge_check_conversions", "adambridge_convert", "adambridge_plan_launches",
     "adambridge_multi_step_noalloc", "adambridge_stream_copy", "adambridge_recycle_device_memory",
-    "adambridge_convert_plane", "adambridge_capabilities",
+    "adambridge_convert_plane", "adambridge_capabilities", "adambridge_cross_entropy_work",
+    "adambridge_cross_entropy", "adambridge_cross_entropy_backward",
 )
 
 
@@ -147,6 +148,9 @@ def open_library(path: Path = LIB_PATH) -> ctypes.CDLL:
         "adambridge_convert_plane": (ctypes.c_int, [ctypes.POINTER(Plane), ctypes.POINTER(Plane), i64, u64,
                                                     ctypes.c_uint32, i32]),
         "adambridge_capabilities": (ctypes.c_uint32, []),
+        "adambridge_cross_entropy_work": (i64, [i64, i64]),
+        "adambridge_cross_entropy": (ctypes.c_int, [vp, i32, vp, i64, i64, i64, vp, vp, vp]),
+        "adambridge_cross_entropy_backward": (ctypes.c_int, [vp, i32, vp, i64, i64, i64, vp, vp, vp]),
     }
     for name in EXPORTS:
         fn = getattr(lib, name)
@@ -350,6 +354,42 @@ class HipKernels:
                                                     0 if seed is None else seed & 0xFFFFFFFF,
                                                     0 if seed is None else CONVERT_STOCHASTIC)
         self._check(rc, "adambridge_convert_plane")
+
+    # -- cross-entropy ---------------------------------------------------------
+
+    def cross_entropy(self, logits: torch.Tensor, target: torch.Tensor, ignore_index: int
+                      ) -> tuple[torch.Tensor, torch.Tensor]:
+        """Summed cross-entropy of contiguous [rows, vocab] float32 or bfloat16 logits against int64
+        classes, on the current stream (adambridge_cross_entropy): the FP32 sum and the per-row
+        statistics its gradient takes."""
+        rows, vocab = logits.shape
+        nbytes = self._lib.adambridge_cross_entropy_work(rows, vocab)
+        if nbytes < 0:
+            self._check(nbytes, "adambridge_cross_entropy_work")
+        work = torch.empty(nbytes // 4, dtype=torch.float32, device=logits.device)
+        stats = torch.empty(rows, 2, dtype=torch.float32, device=logits.device)
+        loss = torch.empty((), dtype=torch.float32, device=logits.device)
+        with torch.cuda.device(logits.device):
+            self._lib.adambridge_set_stream(torch.cuda.current_stream(logits.device).cuda_stream)
+            rc = self._lib.adambridge_cross_entropy(logits.data_ptr(), _DTYPE_CODES[logits.dtype], target.data_ptr(), rows,
+                                                    vocab, ignore_index, work.data_ptr(), stats.data_ptr(),
+                                                    loss.data_ptr())
+        self._check(rc, "adambridge_cross_entropy")
+        return loss, stats
+
+    def cross_entropy_backward(self, logits: torch.Tensor, target: torch.Tensor, ignore_index: int,
+                               stats: torch.Tensor, gout: torch.Tensor) -> torch.Tensor:
+        """The gradient of :meth:`cross_entropy`'s sum with respect to the logits, times ``gout`` (an FP32
+        scalar on the device), in the logits' type (adambridge_cross_entropy_backward)."""
+        rows, vocab = logits.shape
+        grad = torch.empty_like(logits)
+        with torch.cuda.device(logits.device):
+            self._lib.adambridge_set_stream(torch.cuda.current_stream(logits.device).cuda_stream)
+            rc = self._lib.adambridge_cross_entropy_backward(
+                logits.data_ptr(), _DTYPE_CODES[logits.dtype], target.data_ptr(), rows, vocab, ignore_index,
+                stats.data_ptr(), gout.data_ptr(), grad.data_ptr())
+        self._check(rc, "adambridge_cross_entropy_backward")
+        return grad
 
     def fused_adamw(self, master: torch.Tensor, grad: torch.Tensor, m: torch.Tensor, v: torch.Tensor,
                     out: torch.Tensor | None, hp: HParams, lo: int, hi: int) -> None:

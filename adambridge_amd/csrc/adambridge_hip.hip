@@ -46,6 +46,7 @@
 
 #include "../../include/adambridge_hip.h"
 #include "abh_device.hpp"
+#include "abh_host.hpp"
 
 namespace abh {
 

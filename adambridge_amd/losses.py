@@ -4,8 +4,12 @@ The output projection of a large-vocabulary model turns [batch, seq, hidden] act
 [batch, seq, vocab] logits -- gigabytes in FP32 for a 150k vocabulary -- which training then
 keeps for the backward pass.  ``causal_lm_loss`` projects a slice of positions at a time and,
 with gradients enabled, recomputes each slice's logits in the backward pass instead of keeping
-them, so at most one slice of logits exists at once.  Plain PyTorch: this is off the optimizer's
-path and runs wherever the model runs.
+them, so at most one slice of logits exists at once.
+
+On the GPU a slice's cross-entropy and its gradient each are one pass of the library's kernels over
+the logits as the head wrote them (csrc/abh_loss.hip).  Elsewhere, and wherever the slice is being
+traced or differentiated in another way than one backward pass (:func:`_kernels_apply`), it is the
+composition of torch operations, which defines the values.
 """
 
 from __future__ import annotations
@@ -13,17 +17,69 @@ from __future__ import annotations
 from typing import Callable
 
 import torch
+import torch.autograd.forward_ad as forward_ad
 import torch.nn.functional as F
 from torch.utils.checkpoint import checkpoint
+
+from . import _hip
 
 __all__ = ["causal_lm_loss"]
 
 
+_MAX_ROWS = 1 << 23   # adambridge_cross_entropy's
+
+
+def _kernels_apply(logits: torch.Tensor, target: torch.Tensor) -> bool:
+    """Whether the library's cross-entropy takes this slice: plain contiguous tensors of its types on one
+    GPU, and nothing that needs the torch operations themselves -- a trace or compilation, a function
+    transform (vmap, functorch grad), forward-mode derivatives, a mode that observes operations."""
+    if (torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._are_functorch_transforms_active()
+            or forward_ad._current_level >= 0 or torch._C._len_torch_dispatch_stack()
+            or torch._C._len_torch_function_stack()):
+        return False
+    return (type(logits) is torch.Tensor and type(target) is torch.Tensor
+            and logits.is_cuda and target.device == logits.device
+            and logits.dtype in (torch.bfloat16, torch.float32) and target.dtype == torch.int64
+            and logits.dim() == 2 and target.dim() == 1 and target.numel() == logits.shape[0]
+            and logits.is_contiguous() and target.is_contiguous() and not logits.is_neg()
+            and 0 < logits.shape[0] <= _MAX_ROWS and logits.shape[1] > 0
+            and logits.data_ptr() % 16 == 0)   # so that the gradient, a new tensor, shares its alignment
+
+
+class _SliceLoss(torch.autograd.Function):
+    """Summed cross-entropy by the library's kernels.  What is kept for the backward pass is the logits
+    themselves and two floats per row."""
+
+    @staticmethod
+    def forward(ctx, logits, target, ignore_index):
+        loss, stats = _hip.load().cross_entropy(logits, target, ignore_index)
+        ctx.save_for_backward(logits, target, stats)
+        ctx.ignore_index = ignore_index
+        return loss
+
+    @staticmethod
+    def backward(ctx, gout):
+        logits, target, stats = ctx.saved_tensors
+        if torch.is_grad_enabled():   # create_graph: a gradient that is differentiated in turn
+            loss = _torch_loss_sum(logits, target, ctx.ignore_index)
+            return torch.autograd.grad(loss, logits, gout, create_graph=True)[0], None, None
+        return _hip.load().cross_entropy_backward(logits, target, ctx.ignore_index, stats, gout), None, None
+
+
+def _torch_loss_sum(logits: torch.Tensor, target: torch.Tensor, ignore_index: int) -> torch.Tensor:
+    """Summed cross-entropy, logits upcast to FP32."""
+    return F.cross_entropy(logits.float(), target, ignore_index=ignore_index, reduction="sum")
+
+
 def _slice_loss_sum(h: torch.Tensor, target: torch.Tensor, project: Callable[[torch.Tensor], torch.Tensor],
                     ignore_index: int) -> torch.Tensor:
-    """Summed cross-entropy of one slice, logits upcast to FP32."""
-    logits = project(h).float()
-    return F.cross_entropy(logits, target, ignore_index=ignore_index, reduction="sum")
+    """Summed cross-entropy of one slice."""
+    logits = project(h)
+    if not _kernels_apply(logits, target):
+        return _torch_loss_sum(logits, target, ignore_index)
+    if torch.is_grad_enabled() and logits.requires_grad:
+        return _SliceLoss.apply(logits, target, ignore_index)
+    return _hip.load().cross_entropy(logits, target, ignore_index)[0]
 
 
 def causal_lm_loss(hidden_states: torch.Tensor, lm_head: Callable[[torch.Tensor], torch.Tensor],

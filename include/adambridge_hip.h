@@ -433,6 +433,26 @@ ADAMBRIDGE_API int adambridge_stream_copy(const void* src, void* dst, int64_t nb
  * ADAMBRIDGE_ENULL for a NULL array or count < 1, ADAMBRIDGE_EHIP on a HIP failure. */
 ADAMBRIDGE_API int adambridge_check_conversions(uint32_t seed, uint64_t* mismatches, int32_t count);
 
+/* Summed cross-entropy of a slice of logits and its gradient (reference adambridge/losses.py:27-70),
+ * on the calling thread's stream (asynchronous).  logits: rows x vocab values, contiguous
+ * (ADAMBRIDGE_DT_F32 or _BF16); target: one class per row, a row whose target equals ignore_index
+ * counting nothing.  adambridge_cross_entropy writes the sum of the rows' losses to loss[0] and, for
+ * the gradient, two floats per row to stats (the row's maximum and the reciprocal of its sum of
+ * exponentials); work holds adambridge_cross_entropy_work(rows, vocab) bytes of scratch, 8-byte
+ * aligned.  adambridge_cross_entropy_backward writes (softmax - one_hot(target)) * gout[0] to grad, in
+ * the logits' type.  All of it is computed in FP32; sums are taken in a fixed order.  A target
+ * outside [0, vocab) other than ignore_index makes the loss NaN (nothing is read for it).  Returns 0,
+ * ADAMBRIDGE_EBADN (rows outside 1 .. 2^23, vocab < 1), _EMVDTYPE, _ENULL, _EALIGN (grad at another offset
+ * from a 16-byte boundary than logits) or _EHIP; adambridge_cross_entropy_work the bytes, or
+ * ADAMBRIDGE_EBADN. */
+ADAMBRIDGE_API int64_t adambridge_cross_entropy_work(int64_t rows, int64_t vocab);
+ADAMBRIDGE_API int adambridge_cross_entropy(const void* logits, int32_t dtype, const int64_t* target, int64_t rows,
+                                            int64_t vocab, int64_t ignore_index, void* work, float* stats,
+                                            float* loss);
+ADAMBRIDGE_API int adambridge_cross_entropy_backward(const void* logits, int32_t dtype, const int64_t* target,
+                                                     int64_t rows, int64_t vocab, int64_t ignore_index,
+                                                     const float* stats, const float* gout, void* grad);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1,0 +1,151 @@
+"""The library's cross-entropy kernels (csrc/abh_loss.hip) against float64 on the same logits, and
+causal_lm_loss where the kernels must not be taken."""
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+import adambridge_amd as ab
+from adambridge_amd import _hip, losses
+
+pytestmark = pytest.mark.gpu
+IGNORE = -100
+
+
+def _case(rows, vocab, dtype, seed=0, scale=4.0):
+    gen = torch.Generator("cuda").manual_seed(seed)
+    logits = (torch.randn(rows, vocab, generator=gen, device="cuda") * scale).to(dtype)
+    target = torch.randint(0, vocab, (rows,), generator=gen, device="cuda")
+    target[::3] = IGNORE
+    return logits, target
+
+
+def _exact(logits, target, gout):
+    logp = logits.double().log_softmax(1)
+    keep = (target != IGNORE).double()
+    at = target.clamp(min=0)[:, None]
+    terms = -logp.gather(1, at)[:, 0] * keep
+    grad = (logp.exp().scatter_add(1, at, -torch.ones_like(at, dtype=torch.float64))) * keep[:, None] * gout
+    return terms.sum(), terms, grad
+
+
+# one value, less than a 16-byte vector, a head and a tail around the vectors (odd rows start off the
+# 16-byte boundary), one and several workgroups per row, the largest vocabulary
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows,vocab", [(1, 1), (5, 7), (4, 8), (3, 2049), (301, 4099), (2050, 1024), (3, 16389),
+                                        (2, 151936), (33, 50257), (1025, 9)])
+def test_loss_and_gradient_match_float64(rows, vocab, dtype):
+    logits, target = _case(rows, vocab, dtype)
+    k = _hip.load()
+    gout = torch.tensor(0.37, device="cuda")
+    loss, stats = k.cross_entropy(logits, target, IGNORE)
+    grad = k.cross_entropy_backward(logits, target, IGNORE, stats, gout)
+    want, terms, want_grad = _exact(logits, target, 0.37)
+    # the sum of FP32 terms: each off by a few ulp of its log-sum (below 32: 4 x 2^-20), their sum by
+    # the roundings of a lane's rows and the tree
+    assert abs(loss.item() - want.item()) <= rows * 4 * 2.0 ** -20 + abs(want.item()) * 2.0 ** -20
+    # p's relative error: |x - m| <= 48 here, times log2(e), rounded once (2^-24 of it), the exponential and
+    # two products: below 48 x 1.45 x 2^-24 + 2^-21 < 2^-17; then the rounding to the logits' type
+    unit = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -23
+    p = (want_grad - torch.zeros_like(want_grad)).abs()
+    bound = p * unit + 0.37 * logits.double().softmax(1) * 2.0 ** -17 + 1e-38
+    assert ((grad.double() - want_grad).abs() <= bound).all()
+    assert not grad[::3].any()   # ignored rows
+
+
+def test_infinities_nan_and_targets_outside_the_vocabulary():
+    k = _hip.load()
+    gout = torch.ones((), device="cuda")
+    logits = torch.randn(8, 300, device="cuda", generator=torch.Generator("cuda").manual_seed(3))
+    target = torch.arange(8, device="cuda") + 5
+    logits[0, 100:] = -torch.inf
+    logits[1] = -torch.inf
+    logits[2, 7] = torch.nan
+    logits[3, 3] = torch.inf
+    logits[4, :200] = torch.finfo(torch.float32).min
+    logits[5] = torch.finfo(torch.float32).min
+    target[6] = IGNORE
+    logits[6, 9] = torch.nan   # an ignored row's NaN reaches its gradient, as in torch's operations
+    for r in range(8):
+        one, t = logits[r:r + 1].clone().requires_grad_(), target[r:r + 1]
+        want = F.cross_entropy(one, t, ignore_index=IGNORE, reduction="sum")
+        want.backward()
+        loss, stats = k.cross_entropy(one.detach(), t, IGNORE)
+        grad = k.cross_entropy_backward(one.detach(), t, IGNORE, stats, gout)
+        assert torch.allclose(loss, want.detach(), rtol=2e-6, atol=1e-6, equal_nan=True), r
+        assert torch.allclose(grad, one.grad, rtol=1e-5, atol=1e-7, equal_nan=True), r
+    for bad in (300, -1):
+        assert k.cross_entropy(logits[7:], torch.tensor([bad], device="cuda"), IGNORE)[0].isnan()
+
+
+def _problem(dtype=torch.bfloat16, vocab=997, seed=1):
+    gen = torch.Generator("cuda").manual_seed(seed)
+    hidden = torch.randn(2, 40, 64, generator=gen, device="cuda").to(dtype).requires_grad_()
+    head = torch.nn.Linear(64, vocab, bias=False, device="cuda", dtype=dtype)
+    with torch.no_grad():
+        head.weight.normal_(0.0, 0.2, generator=gen)
+    labels = torch.randint(0, vocab, (2, 40), generator=gen, device="cuda")
+    labels[:, :9] = IGNORE
+    return hidden, head, labels
+
+
+def _grads(hidden, head, labels, **kw):
+    hidden.grad = head.weight.grad = None
+    loss = ab.causal_lm_loss(hidden, head, labels, chunk_tokens=32)
+    loss.backward(**kw)
+    return loss.detach(), hidden.grad, head.weight.grad
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_causal_lm_loss_takes_the_kernels_and_agrees_with_torch(dtype, monkeypatch):
+    problem = _problem(dtype)
+    calls = []
+    k = _hip.load()
+    real = k.cross_entropy_backward
+    monkeypatch.setattr(k, "cross_entropy_backward", lambda *a: calls.append(1) or real(*a))
+    got = _grads(*problem)
+    assert len(calls) == 3   # 80 positions, 32 at a time
+    with torch.autograd.graph.save_on_cpu():
+        moved = _grads(*problem)
+    monkeypatch.setattr(losses, "_kernels_apply", lambda *a: False)
+    want = _grads(*problem)
+    # two roundings of the logits' gradient to BF16 (2^-8 apart at most, at random) before the products
+    tol = 2.0 ** -8 if dtype == torch.bfloat16 else 1e-5
+    for a, b, c in zip(got, want, moved):
+        assert (a - b).norm() <= tol * b.norm() and torch.equal(a, c)
+
+
+def test_second_derivatives_and_transforms_use_torch_operations(monkeypatch):
+    hidden, head, labels = _problem(torch.float32, vocab=61)
+    target = torch.zeros(80, dtype=torch.int64, device="cuda")
+    logits = head(hidden.reshape(80, 64)).detach().requires_grad_()
+
+    def second():
+        loss = losses._slice_loss_sum(logits, target, lambda x: x, IGNORE)
+        (g,) = torch.autograd.grad(loss, logits, create_graph=True)
+        return g.detach(), torch.autograd.grad(g.square().sum(), logits)[0]
+
+    got = second()
+    rows = torch.func.vmap(lambda h: losses._slice_loss_sum(h, target[:40], head, IGNORE))(hidden.detach())
+    tangent = torch.func.jvp(lambda x: losses._slice_loss_sum(x, target, lambda y: y, IGNORE), (logits.detach(),),
+                             (torch.ones_like(logits),))[1]
+    monkeypatch.setattr(losses, "_kernels_apply", lambda *a: False)
+    want = second()
+    for a, b in zip(got, want):
+        assert torch.allclose(a, b, rtol=1e-4, atol=1e-6)
+    each = torch.stack([losses._slice_loss_sum(h, target[:40], head, IGNORE) for h in hidden.detach()])
+    assert torch.allclose(rows, each, rtol=1e-5)
+    assert abs(tangent.item()) < 1e-2   # a shift of every logit leaves the loss as it is
+
+
+def test_other_types_and_strides_use_torch_operations():
+    target = torch.zeros(4, dtype=torch.int64, device="cuda")
+    base = torch.randn(4, 66, device="cuda")
+    assert losses._kernels_apply(base, target)
+    assert not losses._kernels_apply(base[:, :64], target)                      # strided rows
+    assert not losses._kernels_apply(base.half(), target)
+    assert not losses._kernels_apply(base, target.int())
+    assert not losses._kernels_apply(base.reshape(-1)[1:-65].view(3, 66), target[:3])   # off the 16-byte boundary
+    assert not losses._kernels_apply(base.cpu(), target.cpu())
+    loss = losses._slice_loss_sum(base.half(), target, lambda x: x, IGNORE)
+    assert torch.allclose(loss, F.cross_entropy(base.half().float(), target, reduction="sum"))
