@@ -19,7 +19,7 @@ from pathlib import Path
 
 import torch
 
-__all__ = ["HipKernels", "HParams", "Group", "Segment", "Plane", "plane_of", "fp24_plane", "load", "LIB_PATH", "DT_NONE", "DT_F32", "DT_BF16",
+__all__ = ["HipKernels", "HParams", "Group", "Segment", "Plane", "State", "Arrays", "plane_of", "fp24_plane", "load", "LIB_PATH", "DT_NONE", "DT_F32", "DT_BF16",
            "DT_FP8", "DT_F24", "DT_PACKED", "DT_PACKED8", "DT_PACKED_LION", "DT_PACKED_F32", "DT_PACKED_F24", "DT_PACKED_LION_F24",
            "DT_PACKED8_F24", "DT_PACKED_LION_F32", "DT_PACKED8_LION", "DT_PACKED_F24_F32", "DT_PACKED_LION_F24_F32", "DT_PACKED8_LION_F24",
            "SEG_OUT_PREVIOUS", "MOMENT_CODES", "MASTER_CODES",
@@ -73,6 +73,19 @@ class Plane(ctypes.Structure):
                 ("dtype", ctypes.c_int32), ("group_log2", ctypes.c_int32)]
 
 
+class State(ctypes.Structure):
+    """adambridge_state: one parameter's interleaved state (no reference counterpart)."""
+    _fields_ = [("data", ctypes.c_void_p), ("m_scale", ctypes.c_void_p), ("v_scale", ctypes.c_void_p),
+                ("n", ctypes.c_int64), ("layout", ctypes.c_int32), ("reserved", ctypes.c_int32)]
+
+
+class Arrays(ctypes.Structure):
+    """adambridge_arrays: a state's separate arrays, None for what a call leaves out."""
+    _fields_ = [("p", ctypes.c_void_p), ("p_lo", ctypes.c_void_p), ("m", ctypes.c_void_p), ("v", ctypes.c_void_p),
+                ("m_scale", ctypes.c_void_p), ("v_scale", ctypes.c_void_p), ("p_dtype", ctypes.c_int32),
+                ("mv_dtype", ctypes.c_int32)]
+
+
 CONVERT_STOCHASTIC = 1
 CAPABILITIES = {"packed_layouts": 0x01, "out_previous": 0x02, "noalloc": 0x04, "convert": 0x08,
                 "convert_plane": 0x10, "stream_copy": 0x20, "fp8_f24_records": 0x40, "lion_f32_records": 0x80,
@@ -107,7 +120,8 @@ EXPORTS = (
     "adambridge_check_conversions", "adambridge_convert", "adambridge_plan_launches",
     "adambridge_multi_step_noalloc", "adambridge_stream_copy", "adambridge_recycle_device_memory",
     "adambridge_convert_plane", "adambridge_capabilities", "adambridge_cross_entropy_work",
-    "adambridge_cross_entropy", "adambridge_cross_entropy_backward",
+    "adambridge_cross_entropy", "adambridge_cross_entropy_backward", "adambridge_unpack_state",
+    "adambridge_pack_state",
 )
 
 
@@ -148,6 +162,8 @@ def open_library(path: Path = LIB_PATH) -> ctypes.CDLL:
         "adambridge_convert_plane": (ctypes.c_int, [ctypes.POINTER(Plane), ctypes.POINTER(Plane), i64, u64,
                                                     ctypes.c_uint32, i32]),
         "adambridge_capabilities": (ctypes.c_uint32, []),
+        "adambridge_unpack_state": (ctypes.c_int, [ctypes.POINTER(State), ctypes.POINTER(Arrays)]),
+        "adambridge_pack_state": (ctypes.c_int, [ctypes.POINTER(State), ctypes.POINTER(Arrays)]),
         "adambridge_cross_entropy_work": (i64, [i64, i64]),
         "adambridge_cross_entropy": (ctypes.c_int, [vp, i32, vp, i64, i64, i64, vp, vp, vp]),
         "adambridge_cross_entropy_backward": (ctypes.c_int, [vp, i32, vp, i64, i64, i64, vp, vp, vp]),
@@ -354,6 +370,17 @@ class HipKernels:
                                                     0 if seed is None else seed & 0xFFFFFFFF,
                                                     0 if seed is None else CONVERT_STOCHASTIC)
         self._check(rc, "adambridge_convert_plane")
+
+    def move_state(self, state: State, arrays: Arrays, device: torch.device, pack: bool) -> None:
+        """Between an interleaved state and separate arrays on ``device``'s current stream, one pass:
+        ``pack`` writes the arrays into the state (adambridge_pack_state), else the state's columns
+        into the arrays (adambridge_unpack_state).  The memory must stay alive until the stream has
+        run it."""
+        fn = self._lib.adambridge_pack_state if pack else self._lib.adambridge_unpack_state
+        with torch.cuda.device(device):
+            self._lib.adambridge_set_stream(torch.cuda.current_stream(device).cuda_stream)
+            rc = fn(ctypes.byref(state), ctypes.byref(arrays))
+        self._check(rc, "adambridge_pack_state" if pack else "adambridge_unpack_state")
 
     # -- cross-entropy ---------------------------------------------------------
 

@@ -18,7 +18,7 @@ from pathlib import Path
 
 PKG = Path(__file__).resolve().parent
 ROOT = PKG.parent
-SOURCES = [PKG / "csrc" / name for name in ("adambridge_hip.hip", "abh_loss.hip")]
+SOURCES = [PKG / "csrc" / name for name in ("adambridge_hip.hip", "abh_state.hip", "abh_loss.hip")]
 LIB = PKG / "libadambridge_hip.so"
 ARCH = os.environ.get("ADAMBRIDGE_HIP_ARCH", "gfx950")
 

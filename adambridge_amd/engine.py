@@ -313,9 +313,11 @@ class UpdateEngine:
     def rebuild(self, slots: list[ParamSlot], precision: str | None = None, masters: list | None = None,
                 moments: list[dict[str, MomentStore] | None] | None = None) -> None:
         """New states for ``slots`` in ``precision`` (default: the engine's), each in the layout that
-        serves it -- one arena per device and layout, as :meth:`initialize`.  ``masters[i]``: checkpoint
-        master weights for slot i, or None to keep its master (a fresh slot: the parameter's value);
-        ``moments[i]``: stores of that precision, or None to re-encode its current moments."""
+        serves it -- one arena per device and layout, as :meth:`initialize`; a state already in that
+        layout is kept and written over.  ``masters[i]``: checkpoint master weights for slot i, or
+        None to keep its master (a fresh slot: the parameter's value); ``moments[i]``: stores of that
+        precision (of any for an interleaved state, which converts them), or None to re-encode its
+        current moments."""
         precision = precision or self.precision
         masters = masters or [None] * len(slots)
         moments = moments or [None] * len(slots)
@@ -327,24 +329,48 @@ class UpdateEngine:
             groups.setdefault((slot.param.device, self.layout_for(slot, precision)), []).append(i)
         for (device, layout), picks in groups.items():
             with torch.cuda.device(device), torch.no_grad():
-                values, params, loads = [], [], []
+                if layout == "separate":
+                    self._rebuild_separate(device, precision, [slots[i] for i in picks], [masters[i] for i in picks],
+                                           [moments[i] for i in picks])
+                    continue
+                # a state of this layout is written into in place; the others are made, in one arena
+                kept = {i: slots[i].state for i in picks if slots[i].state is not None
+                        and slots[i].state.layout == layout and slots[i].state.device == device}
+                fresh = [i for i in picks if i not in kept]
+                states = dict(kept)
+                if fresh:
+                    made = new_states(layout, self.algorithm, precision, self.master_precision, device,
+                                      [slots[i].param.detach().reshape(-1) for i in fresh], self.double_buffer, fill=False)
+                    states.update(zip(fresh, made))
                 for i in picks:
                     slot, old = slots[i], slots[i].state
-                    param = slot.param if self._master_is_param(slot.param) else None
-                    values.append(slot.param.detach().reshape(-1) if param is not None or old is None
-                                  else old.master_fp32())
-                    params.append(param)
-                    held = moments[i]
-                    if held is None:
-                        held = {r: make_store(precision, slot.numel, r, init=old.moment(r).to_fp32(), device=device)
-                                for r in old.roles}
-                    loads.append(held)
-                states = new_states(layout, self.algorithm, precision, self.master_precision, device, values,
-                                    self.double_buffer, params)
-                for i, state, held in zip(picks, states, loads):
-                    state.load(master=masters[i], moments=held)
-                    self._adopt(slots[i], state)
-                    self._ensure_out(slots[i])
+                    master = masters[i]
+                    if master is None and i not in kept:
+                        master = slot.param.detach().reshape(-1) if old is None else old.master_fp32()
+                    held = moments[i] if moments[i] is not None else {r: old.moment(r) for r in old.roles}
+                    states[i].load(master=master, moments=held)
+                    self._adopt(slot, states[i])
+                    self._ensure_out(slot)
+
+    def _rebuild_separate(self, device: torch.device, precision: str, slots: list[ParamSlot], masters: list,
+                          moments: list) -> None:
+        """:meth:`rebuild` for slots whose state is in separate arrays."""
+        values, params, loads = [], [], []
+        for slot, held in zip(slots, moments):
+            old = slot.state
+            param = slot.param if self._master_is_param(slot.param) else None
+            values.append(slot.param.detach().reshape(-1) if param is not None or old is None else old.master_fp32())
+            params.append(param)
+            if held is None:
+                held = {r: make_store(precision, slot.numel, r, init=old.moment(r).to_fp32(), device=device)
+                        for r in old.roles}
+            loads.append(held)
+        states = new_states("separate", self.algorithm, precision, self.master_precision, device, values,
+                            self.double_buffer, params)
+        for slot, state, master, held in zip(slots, states, masters, loads):
+            state.load(master=master, moments=held)
+            self._adopt(slot, state)
+            self._ensure_out(slot)
 
     def _ensure_out(self, slot: ParamSlot) -> None:
         """The write-back buffer of a slot whose updates go there first (deferred write-back, a

@@ -44,7 +44,7 @@ import torch._dynamo  # noqa: F401 -- imported here, not by the first torch.comp
 #                       keeps the frames on the stack alive, which would pin the optimizer being built
 
 from .engine import ParamSlot, SmallGroup, StepStats, UpdateEngine
-from .precision import (_checked, bytes_per_param, canonical_master_precision, canonical_precision,
+from .precision import (FP32Store, _checked, bytes_per_param, canonical_master_precision, canonical_precision,
                         check_master_state, make_store, store_from_state_dict)
 
 __all__ = ["AdamBridge", "LionBridge", "OptiComputeAdamW", "AutoTuneConfig"]
@@ -293,13 +293,18 @@ class _CheckpointReader:
             raise ValueError("checkpoint has no exp_avg_sq (saved by LionBridge?); AdamW needs both moments")
 
     @staticmethod
-    def moment(saved: Any, numel: int, role: str, precision: str, device):
+    def moment(saved: Any, numel: int, role: str, precision: str, device, borrow: bool = False):
         """A saved moment as a store of ``precision``: the torch.optim.AdamW layout (a plain tensor)
-        converted, a store dictionary rebuilt and converted if its precision differs."""
+        converted, a store dictionary rebuilt and converted if its precision differs.  With ``borrow``
+        (an interleaved state packs it next, converting on the way) the store may be of the saved
+        precision and hold the checkpoint's own tensors."""
         if isinstance(saved, torch.Tensor):
-            return make_store(precision, numel, role, init=saved.to(device, torch.float32), device=device)
-        store = store_from_state_dict(saved, numel, role, device=device)
-        if store.precision == precision:
+            values = saved.to(device, torch.float32)
+            if borrow:
+                return FP32Store.wrap(values.detach().reshape(-1).contiguous())
+            return make_store(precision, numel, role, init=values, device=device)
+        store = store_from_state_dict(saved, numel, role, device=device, borrow=borrow)
+        if store.precision == precision or borrow:
             return store
         return make_store(precision, numel, role, init=store.to_fp32(), device=device)
 
@@ -681,8 +686,9 @@ class AdamBridge(torch.optim.Optimizer):
                 slot.step = int(entry["step"])
                 slots.append(slot)
                 masters.append(entry.get("master"))
-                moments.append({role: reader.moment(entry[key], slot.numel, role, self.precision, slot.param.device)
-                                for role, key in keys})
+                borrow = slot.param.is_cuda and self._engine.layout_for(slot) != "separate"
+                moments.append({role: reader.moment(entry[key], slot.numel, role, self.precision, slot.param.device,
+                                                    borrow) for role, key in keys})
         self._engine.rebuild(slots, self.precision, masters, moments)
 
     def close(self) -> None:

@@ -174,6 +174,13 @@ class BF16Store(MomentStore):
     def read(self, lo, hi):
         return self.data[lo:hi].float()
 
+    @classmethod
+    def wrap(cls, data: torch.Tensor) -> "BF16Store":
+        """The store whose values are the flat BF16 tensor ``data`` itself."""
+        store = cls(0, device=data.device)
+        store.numel, store.data = data.numel(), data
+        return store
+
     def write(self, lo, hi, x, seed=None):
         self.data[lo:hi].copy_(F.bf16_encode(_flat_fp32(x, self.device), seed, lo))
 
@@ -201,17 +208,29 @@ class FP8Store(MomentStore):
     def __init__(self, numel: int, role: str, init: torch.Tensor | None = None, block: int = FP8_BLOCK,
                  device=None):
         super().__init__(numel, _home(device, init))
+        self._set_format(role, block)
+        nb = F.fp8_blocks(self.numel, self.block)
+        self.q = torch.zeros(nb * self.block, dtype=self.dtype, device=self.device)
+        self.scale = torch.ones(nb, dtype=torch.float32, device=self.device)
+        if init is not None:
+            self.write(0, self.numel, init)
+
+    @classmethod
+    def wrap(cls, q: torch.Tensor, scale: torch.Tensor, numel: int, role: str, block: int) -> "FP8Store":
+        """The store of ``numel`` values whose codes and scales are the flat tensors ``q`` and ``scale``."""
+        store = cls.__new__(cls)
+        MomentStore.__init__(store, numel, q.device)
+        store._set_format(role, block)
+        store.q, store.scale = q, scale
+        return store
+
+    def _set_format(self, role: str, block: int) -> None:
         if role not in F.FP8_FORMATS:
             raise ValueError(f"role must be 'm' or 'v', got {role!r}")
         self.role, self.block = role, int(block)
         self.format = F.FP8_FORMATS[role]
         self.dtype, self.fmax = self.format.dtype, self.format.fmax
         self.sqrt_domain = self.format.sqrt_domain
-        nb = F.fp8_blocks(self.numel, self.block)
-        self.q = torch.zeros(nb * self.block, dtype=self.dtype, device=self.device)
-        self.scale = torch.ones(nb, dtype=torch.float32, device=self.device)
-        if init is not None:
-            self.write(0, self.numel, init)
 
     def _blocks(self, lo: int, hi: int) -> tuple[int, int]:
         return lo // self.block, -(-hi // self.block)
@@ -260,6 +279,13 @@ class FP24Store(MomentStore):
         if init is not None:
             self.init_from_(init)
 
+    @classmethod
+    def wrap(cls, hi: torch.Tensor, lo: torch.Tensor) -> "FP24Store":
+        """The store whose planes are the flat tensors ``hi`` (bfloat16) and ``lo`` (uint8) themselves."""
+        store = cls(0, device=hi.device)
+        store.numel, store.hi, store.lo = hi.numel(), hi, lo
+        return store
+
     def init_from_(self, src: torch.Tensor) -> None:
         """Planes from ``src``: BF16 bits are exact (low plane zero); other values round to nearest even,
         INIT_CHUNK elements at a time."""
@@ -305,6 +331,23 @@ def make_store(precision: str, numel: int, role: str, init: torch.Tensor | None 
     if precision == "fp8":
         return FP8Store(numel, role, init, device=device)
     return _MOMENT_STORES[precision](numel, init, device=device)
+
+
+def blank_store(precision: str, numel: int, role: str, device) -> MomentStore:
+    """A store ('fp32', 'bf16', 'fp8' or 'fp24') whose values the caller is about to write, all of them:
+    its memory is not cleared first.  (An FP8 store of no elements keeps its one block of zero codes.)"""
+    if not numel:
+        return make_master(precision, numel, device=device) if precision == "fp24" else \
+            make_store(precision, numel, role, device=device)
+    if precision == "fp24":
+        return FP24Store.wrap(torch.empty(numel, dtype=torch.bfloat16, device=device),
+                              torch.empty(numel, dtype=torch.uint8, device=device))
+    if precision == "fp8":
+        nb = F.fp8_blocks(numel)
+        return FP8Store.wrap(torch.empty(nb * FP8_BLOCK, dtype=F.FP8_FORMATS[role].dtype, device=device),
+                             torch.empty(nb, dtype=torch.float32, device=device), numel, role, FP8_BLOCK)
+    dtype = torch.float32 if precision == "fp32" else torch.bfloat16
+    return _MOMENT_STORES[precision].wrap(torch.empty(numel, dtype=dtype, device=device))
 
 
 def make_master(precision: str, numel: int, init: torch.Tensor | None = None, device=None) -> MomentStore:
@@ -364,15 +407,23 @@ def load_master_(store: MomentStore, saved: Any) -> None:
     store.write(0, store.numel, master_to_fp32(saved, store.numel, store.device))
 
 
-def store_from_state_dict(state: Any, numel: int, role: str, device=None) -> MomentStore:
+def _borrowed(t: torch.Tensor, dtype: torch.dtype, device) -> bool:
+    """Whether a checkpoint's tensor can stand in a store as it is: its type, on ``device``, contiguous."""
+    return t.dtype == dtype and device is not None and t.device == torch.device(device) and t.is_contiguous()
+
+
+def store_from_state_dict(state: Any, numel: int, role: str, device=None, borrow: bool = False) -> MomentStore:
     """A moment store rebuilt from its checkpoint dictionary, every field validated first.  An FP8
-    store saved for the other role is decoded in its own format and re-encoded in ``role``'s."""
+    store saved for the other role is decoded in its own format and re-encoded in ``role``'s.  With
+    ``borrow`` the store may hold the checkpoint's own tensors (for a caller that only reads it)."""
     kind = state.get("precision") if isinstance(state, dict) else None
     if kind not in PRECISIONS:
         raise ValueError("checkpoint moment store has unknown precision "
                          f"{kind if isinstance(state, dict) else state!r}")
     if kind != "fp8":
         data = _tensor_of(state.get("data"), numel, f"{kind} moments")
+        if borrow and _borrowed(data, torch.float32 if kind == "fp32" else torch.bfloat16, device):
+            return _MOMENT_STORES[kind].wrap(data.detach().reshape(-1))
         store = make_store(kind, numel, role, device=device)
         store.data.copy_(data.reshape(-1))
         return store
@@ -384,6 +435,9 @@ def store_from_state_dict(state: Any, numel: int, role: str, device=None) -> Mom
     nb = F.fp8_blocks(numel, block)
     codes = _tensor_of(state.get("q"), nb * block, "FP8 codes")
     scales = _tensor_of(state.get("scale"), nb, "FP8 scales")
+    if borrow and saved_role == role and _borrowed(codes, F.FP8_FORMATS[role].dtype, device) \
+            and _borrowed(scales, torch.float32, device):
+        return FP8Store.wrap(codes.detach().reshape(-1), scales.detach().reshape(-1), numel, role, block)
     store = FP8Store(numel, saved_role, block=block, device=device)
     store.q.copy_(codes.reshape(-1))
     store.scale.copy_(scales.reshape(-1))

@@ -45,7 +45,8 @@ import torch
 
 from . import _hip
 from . import formats as F
-from .precision import BF16Store, FP8Store, FP24Store, FP32Store, MomentStore, load_master_, make_master, make_store
+from .precision import (BF16Store, FP8Store, FP24Store, FP32Store, MomentStore, blank_store, load_master_, make_master,
+                        make_store)
 
 __all__ = ["ParamState", "SeparateState", "PairState", "AdamRecordState", "LionRecordState", "F32RecordState",
            "F24RecordState", "LionF24RecordState", "AdamF24RecordState", "LionF32RecordState", "LionFP8RecordState", "F24F32RecordState", "LionF24F32RecordState", "LionFP8F24RecordState", "choose_layout", "new_state", "new_states",
@@ -323,22 +324,84 @@ class _Interleaved(ParamState):
     # The master column, the plane-conversion kernel's view of it: (stride in bytes, log2 of the
     # elements per group) of an FP32 master; the FP24-master and FP8-record layouts override master_plane.
     PLANE: tuple[int, int] = (0, 0)
+    CODE = _hip.DT_NONE   # the layout's p_dtype
+    scales: dict[str, torch.Tensor] = {}   # FP8 layouts: each moment's block scales
 
     def master_plane(self):
         stride, log2 = self.PLANE
         return _hip.Plane(self.current.data_ptr(), None, stride, _hip.DT_F32, log2)
 
-    def _load_master(self, master: Any) -> None:
-        """Checkpoint master weights or plain values into the master column: on the device one pass
-        of the plane-conversion kernel (FP24 rounds to nearest; padding slots keep their bits), in
-        host memory a torch copy."""
-        if self.device.type != "cuda":
-            self._put("p", _as_master_values(master, self.numel, self.device))
-            return
-        src, keep = _master_source(master, self.numel, self.device)   # keep: alive until enqueued
+    # On the device the columns go to and from separate arrays in one pass of the library's kernels
+    # (adambridge_unpack_state, adambridge_pack_state); in host memory through the strided views.
+
+    def _move(self, arrays: _hip.Arrays, pack: bool) -> None:
         if self.numel:
-            F.convert_plane(src, self.master_plane(), self.numel, self.device)
-        del keep   # memory made on this stream and freed to it: reused only after the copy
+            state = _hip.State(self.current.data_ptr(), _ptr(self.scales.get("m")), _ptr(self.scales.get("v")),
+                               self.numel, self.CODE, 0)
+            _hip.load().move_state(state, arrays, self.device, pack)
+
+    def _unpacked(self, master: bool, roles: tuple[str, ...]) -> tuple[MomentStore | None, dict[str, MomentStore]]:
+        """The master and the moments ``roles`` as new stores of the layout's own formats, bit for bit."""
+        arrays = _hip.Arrays(mv_dtype=_hip.MOMENT_CODES[self.precision], p_dtype=_hip.MASTER_CODES[self.master_precision])
+        held = blank_store(self.master_precision, self.numel, "m", self.device) if master else None
+        if held is not None:
+            values, low = held.native_buffers
+            arrays.p, arrays.p_lo = values.data_ptr(), _ptr(low)
+        stores = {r: blank_store(self.precision, self.numel, r, self.device) for r in roles}
+        for r, store in stores.items():
+            values, scale = store.native_buffers
+            setattr(arrays, r, values.data_ptr())
+            setattr(arrays, r + "_scale", _ptr(scale))
+        self._move(arrays, pack=False)
+        return held, stores
+
+    def _packed(self, master: Any, moments: dict[str, MomentStore]) -> None:
+        """Master weights or values and moment stores (of any precision) into the state: one pass, or one
+        per format the moments are stored in."""
+        arrays, keep = _hip.Arrays(), []
+        if master is not None:
+            plane, keep = _master_source(master, self.numel, self.device)
+            arrays.p, arrays.p_lo, arrays.p_dtype = plane.data, plane.lo, plane.dtype
+        by_format: dict[str, dict[str, MomentStore]] = {}
+        for role in self.roles:
+            if role in moments:
+                store = _kernel_store(moments[role], role, self.device)
+                by_format.setdefault(store.precision, {})[role] = store
+        for precision, stores in by_format.items() or [("fp32", {})]:
+            arrays.mv_dtype = _hip.MOMENT_CODES[precision]
+            for role, store in stores.items():
+                values, scale = store.native_buffers
+                setattr(arrays, role, values.data_ptr())
+                setattr(arrays, role + "_scale", _ptr(scale))
+            self._move(arrays, pack=True)
+            arrays = _hip.Arrays()
+        del keep, by_format   # read by then in stream order: their memory is freed to the stream they are on
+
+    def moment(self, role):
+        if self.device.type == "cuda":
+            return self._unpacked(False, (role,))[1][role]
+        return self._host_moment(role)
+
+    def export(self, host=False):
+        if self.device.type != "cuda":
+            return super().export(host)
+        master, stores = self._unpacked(True, self.roles)
+        out = {"master": master.data if isinstance(master, FP32Store) else master.state_dict()}
+        for role, key in zip(self.roles, ("exp_avg", "exp_avg_sq")):
+            out[key] = stores[role].state_dict()
+        return _on_host(out) if host else out
+
+    def load(self, master=None, moments=None):
+        if self.device.type == "cuda":
+            self._packed(master, moments or {})
+        else:
+            self._host_load(master, moments)
+
+    def _host_moment(self, role: str) -> MomentStore:
+        raise NotImplementedError
+
+    def _host_load(self, master: Any, moments: dict[str, MomentStore] | None) -> None:
+        raise NotImplementedError
 
     def master_fp32(self):
         if self.device.type != "cuda":
@@ -359,6 +422,7 @@ class PairState(_Interleaved):
     v[2k] | v[2k+1] << 16} (ADAMBRIDGE_DT_PACKED)."""
 
     layout = "pairs"
+    CODE = _hip.DT_PACKED
     precision = "bf16"
     PLANE = (16, 1)   # element i's master at 16 (i >> 1) + 4 (i & 1)
 
@@ -375,7 +439,7 @@ class PairState(_Interleaved):
     def bind(self, seg):
         seg.p, seg.p_lo = self.current.data_ptr(), _ptr(self.target)
         seg.m = seg.v = seg.m_scale = seg.v_scale = None
-        seg.p_dtype, seg.mv_dtype = _hip.DT_PACKED, _hip.DT_BF16
+        seg.p_dtype, seg.mv_dtype = self.CODE, _hip.DT_BF16
 
     def _column(self, role):
         if role == "p":
@@ -383,14 +447,14 @@ class PairState(_Interleaved):
         k = 4 if role == "m" else 6
         return self.current.view(torch.bfloat16)[:, k:k + 2]
 
-    def moment(self, role):
+    def _host_moment(self, role):
         store = BF16Store(self.numel, device=self.device)
         store.data.copy_(self._column(role).reshape(-1)[: self.numel])
         return store
 
-    def load(self, master=None, moments=None):
+    def _host_load(self, master, moments):
         if master is not None:
-            self._load_master(master)
+            self._put("p", _as_master_values(master, self.numel, self.device))
         for role, store in (moments or {}).items():
             self._put(role, _bf16_bits(store, self.device))
 
@@ -404,6 +468,7 @@ class LionRecordState(_Interleaved):
     values, each in element order (ADAMBRIDGE_DT_PACKED_LION)."""
 
     layout = "lion-records"
+    CODE = _hip.DT_PACKED_LION
     precision = "bf16"
     PLANE = (1536, 8)
 
@@ -420,21 +485,21 @@ class LionRecordState(_Interleaved):
     def bind(self, seg):
         seg.p, seg.p_lo = self.current.data_ptr(), _ptr(self.target)
         seg.m = seg.v = seg.m_scale = seg.v_scale = None
-        seg.p_dtype, seg.mv_dtype = _hip.DT_PACKED_LION, _hip.DT_BF16
+        seg.p_dtype, seg.mv_dtype = self.CODE, _hip.DT_BF16
 
     def _column(self, role):
         if role == "p":
             return self.current[:, :1024].view(torch.float32)
         return self.current[:, 1024:].view(torch.bfloat16)
 
-    def moment(self, role):
+    def _host_moment(self, role):
         store = BF16Store(self.numel, device=self.device)
         store.data.copy_(self._column("m").reshape(-1)[: self.numel])
         return store
 
-    def load(self, master=None, moments=None):
+    def _host_load(self, master, moments):
         if master is not None:
-            self._load_master(master)
+            self._put("p", _as_master_values(master, self.numel, self.device))
         if moments and "m" in moments:
             self._put("m", _bf16_bits(moments["m"], self.device))
 
@@ -447,6 +512,7 @@ class F32RecordState(_Interleaved):
     256 m, then the 256 v values, each in element order (ADAMBRIDGE_DT_PACKED_F32)."""
 
     layout = "f32-records"
+    CODE = _hip.DT_PACKED_F32
     precision = "fp32"
     PLANE = (3072, 8)
 
@@ -463,18 +529,18 @@ class F32RecordState(_Interleaved):
     def bind(self, seg):
         seg.p, seg.p_lo = self.current.data_ptr(), _ptr(self.target)
         seg.m = seg.v = seg.m_scale = seg.v_scale = None
-        seg.p_dtype, seg.mv_dtype = _hip.DT_PACKED_F32, _hip.DT_F32
+        seg.p_dtype, seg.mv_dtype = self.CODE, _hip.DT_F32
 
     def _column(self, role):
         k = {"p": 0, "m": 1, "v": 2}[role]
         return self.current[:, 1024 * k:1024 * (k + 1)].view(torch.float32)
 
-    def moment(self, role):
+    def _host_moment(self, role):
         return FP32Store(self.numel, init=self._column(role).reshape(-1)[: self.numel], device=self.device)
 
-    def load(self, master=None, moments=None):
+    def _host_load(self, master, moments):
         if master is not None:
-            self._load_master(master)
+            self._put("p", _as_master_values(master, self.numel, self.device))
         for role, store in (moments or {}).items():
             self._put(role, store.to_fp32().to(self.device))
 
@@ -487,6 +553,7 @@ class LionF32RecordState(F32RecordState):
     values, each in element order (ADAMBRIDGE_DT_PACKED_LION_F32)."""
 
     layout = "lion-f32-records"
+    CODE = _hip.DT_PACKED_LION_F32
     RECORD = 2048
     PLANE = (2048, 8)
 
@@ -502,7 +569,7 @@ class LionF32RecordState(F32RecordState):
 
     def bind(self, seg):
         super().bind(seg)
-        seg.p_dtype = _hip.DT_PACKED_LION_F32
+        seg.p_dtype = self.CODE
 
     def _column(self, role):
         k = {"p": 0, "m": 1}[role]
@@ -518,6 +585,7 @@ class F24RecordState(_Interleaved):
     order (ADAMBRIDGE_DT_PACKED_F24)."""
 
     layout = "f24-records"
+    CODE = _hip.DT_PACKED_F24
     precision = "bf16"
     master_precision = "fp24"
 
@@ -534,7 +602,7 @@ class F24RecordState(_Interleaved):
     def bind(self, seg):
         seg.p, seg.p_lo = self.current.data_ptr(), _ptr(self.target)
         seg.m = seg.v = seg.m_scale = seg.v_scale = None
-        seg.p_dtype, seg.mv_dtype = _hip.DT_PACKED_F24, _hip.DT_BF16
+        seg.p_dtype, seg.mv_dtype = self.CODE, _hip.DT_BF16
 
     def _column(self, role):
         """'p' the hi plane (BF16 bits), 'lo' the lo plane (uint8), 'm' / 'v' the moments (BF16)."""
@@ -568,20 +636,17 @@ class F24RecordState(_Interleaved):
     def export_master(self):
         return self._planes().state_dict()
 
-    def moment(self, role):
+    def _host_moment(self, role):
         store = BF16Store(self.numel, device=self.device)
         store.data.copy_(self._column(role).reshape(-1)[: self.numel])
         return store
 
-    def load(self, master=None, moments=None):
+    def _host_load(self, master, moments):
         if master is not None:
-            if self.device.type == "cuda":
-                self._load_master(master)   # FP24 planes bit for bit; other values rounded to nearest
-            else:
-                planes = FP24Store(self.numel, device=self.device)
-                load_master_(planes, master)   # FP24 planes as they are; other values rounded to nearest
-                self._put("p", planes.hi)
-                self._put("lo", planes.lo)
+            planes = FP24Store(self.numel, device=self.device)
+            load_master_(planes, master)   # FP24 planes as they are; other values rounded to nearest
+            self._put("p", planes.hi)
+            self._put("lo", planes.lo)
         for role, store in (moments or {}).items():
             self._put(role, _bf16_bits(store, self.device))
 
@@ -601,6 +666,7 @@ class F24F32RecordState(F24RecordState):
     order (ADAMBRIDGE_DT_PACKED_F24_F32)."""
 
     layout = "f24-f32-records"
+    CODE = _hip.DT_PACKED_F24_F32
     precision = "fp32"
     RECORD = 2816   # master_plane's record stride too
 
@@ -616,7 +682,7 @@ class F24F32RecordState(F24RecordState):
 
     def bind(self, seg):
         super().bind(seg)
-        seg.p_dtype, seg.mv_dtype = _hip.DT_PACKED_F24_F32, _hip.DT_F32
+        seg.p_dtype, seg.mv_dtype = self.CODE, _hip.DT_F32
 
     def _column(self, role):
         """'p' the hi plane (BF16 bits), 'lo' the lo plane (uint8), 'm' / 'v' the moments (FP32)."""
@@ -625,11 +691,11 @@ class F24F32RecordState(F24RecordState):
         k = {"m": 768, "v": 1792}[role]
         return self.current[:, k:k + 1024].view(torch.float32)
 
-    def moment(self, role):
+    def _host_moment(self, role):
         return FP32Store(self.numel, init=self._column(role).reshape(-1)[: self.numel], device=self.device)
 
-    def load(self, master=None, moments=None):
-        super().load(master)
+    def _host_load(self, master, moments):
+        super()._host_load(master, None)
         for role, store in (moments or {}).items():
             self._put(role, store.to_fp32().to(self.device))
 
@@ -639,6 +705,7 @@ class LionF24RecordState(F24RecordState):
     the 256 low bytes and the 256 m values, each in element order (ADAMBRIDGE_DT_PACKED_LION_F24)."""
 
     layout = "lion-f24-records"
+    CODE = _hip.DT_PACKED_LION_F24
     RECORD = 1280   # master_plane's record stride too
 
     def __init__(self, numel, device, double_buffer: bool = False, memory: list[torch.Tensor] | None = None):
@@ -653,7 +720,7 @@ class LionF24RecordState(F24RecordState):
 
     def bind(self, seg):
         super().bind(seg)
-        seg.p_dtype = _hip.DT_PACKED_LION_F24
+        seg.p_dtype = self.CODE
 
     def window(self, lo, hi):
         w = super().window(lo, hi)
@@ -667,6 +734,7 @@ class LionF24F32RecordState(LionF24RecordState):
     (ADAMBRIDGE_DT_PACKED_LION_F24_F32)."""
 
     layout = "lion-f24-f32-records"
+    CODE = _hip.DT_PACKED_LION_F24_F32
     precision = "fp32"
     RECORD = 1792   # master_plane's record stride too
 
@@ -676,7 +744,7 @@ class LionF24F32RecordState(LionF24RecordState):
 
     def bind(self, seg):
         super().bind(seg)
-        seg.p_dtype, seg.mv_dtype = _hip.DT_PACKED_LION_F24_F32, _hip.DT_F32
+        seg.p_dtype, seg.mv_dtype = self.CODE, _hip.DT_F32
 
     def _column(self, role):
         """'p' the hi plane (BF16 bits), 'lo' the lo plane (uint8), 'm' the moment (FP32)."""
@@ -684,11 +752,11 @@ class LionF24F32RecordState(LionF24RecordState):
             return self.current[:, 768:1792].view(torch.float32)
         return super()._column(role)
 
-    def moment(self, role):
+    def _host_moment(self, role):
         return FP32Store(self.numel, init=self._column(role).reshape(-1)[: self.numel], device=self.device)
 
-    def load(self, master=None, moments=None):
-        F24RecordState.load(self, master)
+    def _host_load(self, master, moments):
+        F24RecordState._host_load(self, master, None)
         for role, store in (moments or {}).items():
             self._put(role, store.to_fp32().to(self.device))
 
@@ -700,6 +768,7 @@ class AdamRecordState(_Interleaved):
     FP32 block-scale array per moment.  Updated in place."""
 
     layout = "fp8-records"
+    CODE = _hip.DT_PACKED8
     precision = "fp8"
 
     def __init__(self, numel, device, double_buffer: bool = False, memory: list[torch.Tensor] | None = None):
@@ -716,7 +785,7 @@ class AdamRecordState(_Interleaved):
     def bind(self, seg):
         seg.p, seg.p_lo, seg.m, seg.v = self.current.data_ptr(), None, None, None
         seg.m_scale, seg.v_scale = self.scales["m"].data_ptr(), self.scales["v"].data_ptr()
-        seg.p_dtype, seg.mv_dtype = _hip.DT_PACKED8, _hip.DT_FP8
+        seg.p_dtype, seg.mv_dtype = self.CODE, _hip.DT_FP8
 
     def _column(self, role):
         if role == "p":   # [block, lane, half, j] = element 128 block + 8 lane + 4 half + j
@@ -730,15 +799,15 @@ class AdamRecordState(_Interleaved):
     def _codes(self, role: str) -> torch.Tensor:
         return self._column(role).reshape(-1).view(F.FP8_FORMATS[role].dtype)
 
-    def moment(self, role):
+    def _host_moment(self, role):
         store = FP8Store(self.numel, role, device=self.device)
         store.q.copy_(self._codes(role))
         store.scale.copy_(self.scales[role])
         return store
 
-    def load(self, master=None, moments=None):
+    def _host_load(self, master, moments):
         if master is not None:
-            self._load_master(master)
+            self._put("p", _as_master_values(master, self.numel, self.device))
         for role, store in (moments or {}).items():
             if not isinstance(store, FP8Store) or store.role != role or store.block != F.FP8_BLOCK:
                 store = FP8Store(self.numel, role, init=store.to_fp32(), device=self.device)
@@ -767,6 +836,7 @@ class AdamF24RecordState(AdamRecordState):
     392 + 16l -- plus an FP32 block-scale array per moment.  Updated in place."""
 
     layout = "fp8-f24-records"
+    CODE = _hip.DT_PACKED8_F24
     master_precision = "fp24"
     RECORD = 640
 
@@ -783,7 +853,7 @@ class AdamF24RecordState(AdamRecordState):
 
     def bind(self, seg):
         super().bind(seg)
-        seg.p_dtype = _hip.DT_PACKED8_F24
+        seg.p_dtype = self.CODE
 
     def _column(self, role):
         """'p' the hi plane (BF16 bits), 'lo' the lo plane (uint8), 'm' / 'v' the codes, in element order."""
@@ -809,14 +879,13 @@ class AdamF24RecordState(AdamRecordState):
     def export_master(self):
         return self._planes().state_dict()
 
-    def load(self, master=None, moments=None):
-        if master is not None and self.device.type != "cuda":
+    def _host_load(self, master, moments):
+        if master is not None:
             planes = FP24Store(self.numel, device=self.device)
             load_master_(planes, master)   # FP24 planes as they are; other values rounded to nearest
             self._put("p", planes.hi)
             self._put("lo", planes.lo)
-            master = None
-        super().load(master, moments)   # on the device: FP24 planes bit for bit, other values to nearest
+        super()._host_load(None, moments)
 
     def footprint(self):
         return 3 * self.numel, self.current.nbytes - 3 * self.numel + sum(s.nbytes for s in self.scales.values())
@@ -834,6 +903,7 @@ class LionFP8RecordState(AdamRecordState):
     the FP32 m block scales.  Updated in place."""
 
     layout = "lion-fp8-records"
+    CODE = _hip.DT_PACKED8_LION
     RECORD = 640   # master_plane's record stride too
 
     def __init__(self, numel, device, double_buffer: bool = False, memory: list[torch.Tensor] | None = None):
@@ -850,7 +920,7 @@ class LionFP8RecordState(AdamRecordState):
     def bind(self, seg):
         seg.p, seg.p_lo, seg.m, seg.v = self.current.data_ptr(), None, None, None
         seg.m_scale, seg.v_scale = self.scales["m"].data_ptr(), None
-        seg.p_dtype, seg.mv_dtype = _hip.DT_PACKED8_LION, _hip.DT_FP8
+        seg.p_dtype, seg.mv_dtype = self.CODE, _hip.DT_FP8
 
     def _column(self, role):
         if role == "p":
@@ -873,6 +943,7 @@ class LionFP8F24RecordState(AdamF24RecordState):
     in place."""
 
     layout = "lion-fp8-f24-records"
+    CODE = _hip.DT_PACKED8_LION_F24
     RECORD = 512   # master_plane's record stride too
 
     def __init__(self, numel, device, double_buffer: bool = False, memory: list[torch.Tensor] | None = None):
@@ -889,7 +960,7 @@ class LionFP8F24RecordState(AdamF24RecordState):
     def bind(self, seg):
         seg.p, seg.p_lo, seg.m, seg.v = self.current.data_ptr(), None, None, None
         seg.m_scale, seg.v_scale = self.scales["m"].data_ptr(), None
-        seg.p_dtype, seg.mv_dtype = _hip.DT_PACKED8_LION_F24, _hip.DT_FP8
+        seg.p_dtype, seg.mv_dtype = self.CODE, _hip.DT_FP8
 
     def _column(self, role):
         if role == "m":
@@ -907,6 +978,17 @@ def _bf16_bits(store: MomentStore, device) -> torch.Tensor:
     if isinstance(store, BF16Store):
         return store.data.to(device)
     return F.bf16_encode(store.to_fp32().to(device))
+
+
+def _kernel_store(store: MomentStore, role: str, device) -> MomentStore:
+    """``store`` as the packing kernel reads it for moment ``role``: itself, on ``device``, where its
+    format is one of the kernel's (FP8: 128-element blocks of the same role), else its FP32 values."""
+    foreign = isinstance(store, FP8Store) and (store.block != F.FP8_BLOCK or store.role != role)
+    if foreign:
+        return FP32Store.wrap(store.to_fp32().to(device).contiguous())
+    if store.device != torch.device(device):
+        return _moved(store, device)
+    return store
 
 
 # -------------------------------------------------------------------- building
@@ -940,16 +1022,38 @@ def arena_plan(layout: str, sizes: list[int], double_buffer: bool = False) -> tu
     return offsets, -(-total // SMALL_ALIGN) * SMALL_ALIGN
 
 
+def _cached(nbytes: int, device: torch.device) -> bool:
+    """Whether torch's allocator holds a free block that an allocation of ``nbytes`` on the current stream
+    will come from (then no memory is asked of the driver)."""
+    if torch.cuda.memory_reserved(device) - torch.cuda.memory_allocated(device) < nbytes:
+        return False
+    stream = torch.cuda.current_stream(device).cuda_stream
+    try:
+        segments = torch.cuda.memory_snapshot()
+    except RuntimeError:   # an allocator that keeps no record
+        return False
+    return any(block["state"] == "inactive" and block["size"] >= nbytes
+               for seg in segments if seg["device"] == device.index and seg["stream"] == stream
+               and tuple(seg.get("segment_pool_id", (0, 0))) == (0, 0) for block in seg["blocks"])
+
+
 def _place(nbytes: int, device, place: bool) -> None:
-    """Before allocating ``nbytes`` of state: an allocate/free of that size (see new_states)."""
-    if place and RECYCLE_MIN_BYTES is not None and nbytes >= RECYCLE_MIN_BYTES:
-        _hip.load().recycle_device_memory(nbytes, torch.device(device))   # placement only: failure is harmless
+    """Before allocating ``nbytes`` of state: an allocate/free of that size (see new_states), unless the
+    allocation will not reach the driver.  The driver clears what it hands out, at 38 GB/s once its
+    cleared memory is used up: a state of 0.9 GB made again and again from cached memory took 24 ms
+    each time for an allocate/free that placed nothing."""
+    if not place or RECYCLE_MIN_BYTES is None or nbytes < RECYCLE_MIN_BYTES:
+        return
+    device = torch.device(device)
+    if device.type == "cuda" and _cached(nbytes, device):
+        return
+    _hip.load().recycle_device_memory(nbytes, device)   # placement only: failure is harmless
 
 
 def new_states(layout: str, algorithm: str, precision: str, master_precision: str, device,
                masters: list[torch.Tensor], double_buffer: bool = False,
                master_params: list[torch.Tensor | None] | None = None, place: bool = True,
-               memory: list[list[torch.Tensor]] | None = None) -> list[ParamState]:
+               memory: list[list[torch.Tensor]] | None = None, fill: bool = True) -> list[ParamState]:
     """Fresh states for several parameters on one device: master from ``masters[i]`` (any dtype;
     FP24 rounds to nearest) or, in the separate layout, the FP32 parameter ``master_params[i]`` itself;
     moments zero, FP8 scales one.
@@ -966,7 +1070,8 @@ def new_states(layout: str, algorithm: str, precision: str, master_precision: st
     update 3-4% slower; measured on MI355X, cause unknown).  The allocate/free holds no more memory
     than the state; it waits for the device to go idle (the free does), so ``place=False`` skips it
     where that would stall a pipeline.  ``memory``: zeroed buffers of an arena made earlier (arena_memory), one list
-    per state, used instead of a new arena (interleaved layouts)."""
+    per state, used instead of a new arena (interleaved layouts).  ``fill=False`` leaves an
+    interleaved state's master at zero, for a caller that loads all of it next."""
     roles = ("m",) if algorithm == "lion" else ("m", "v")
     if layout == "separate":
         # the stores are allocations of their own; the same placement step covers them all at once
@@ -994,7 +1099,8 @@ def new_states(layout: str, algorithm: str, precision: str, master_precision: st
     states = []
     for n, mem, values in zip(sizes, memory, masters):
         state = cls(n, device, double_buffer, memory=mem)
-        state.load(master=values.detach().reshape(-1))   # bf16 or fp32, read as it is by the conversion
+        if fill:
+            state.load(master=values.detach().reshape(-1))   # bf16 or fp32, read as it is by the kernel
         states.append(state)
     return states
 

@@ -433,6 +433,44 @@ ADAMBRIDGE_API int adambridge_stream_copy(const void* src, void* dst, int64_t nb
  * ADAMBRIDGE_ENULL for a NULL array or count < 1, ADAMBRIDGE_EHIP on a HIP failure. */
 ADAMBRIDGE_API int adambridge_check_conversions(uint32_t seed, uint64_t* mismatches, int32_t count);
 
+/* One parameter's interleaved state: layout (a p_dtype of the interleaved layouts above), its
+ * buffer (16-byte aligned) and, for FP8 moments, its block scales. */
+typedef struct adambridge_state {
+    void* data;
+    float* m_scale;
+    float* v_scale;
+    int64_t n;
+    int32_t layout;
+    int32_t reserved;
+} adambridge_state;
+
+/* The same state in separate device arrays of n elements, NULL for what a call leaves out: the
+ * master (ADAMBRIDGE_DT_F32, or DT_F24 with its low bytes in p_lo) and the moments in mv_dtype
+ * (FP8: codes padded to whole 128-element blocks, and a scale per block). */
+typedef struct adambridge_arrays {
+    void* p;
+    uint8_t* p_lo;
+    void* m;
+    void* v;
+    float* m_scale;
+    float* v_scale;
+    int32_t p_dtype;
+    int32_t mv_dtype;
+} adambridge_arrays;
+
+/* No counterpart in the reference, whose state is in separate arrays.  adambridge_unpack_state
+ * copies a state's columns bit for bit into arrays of the layout's own types (a checkpoint);
+ * adambridge_pack_state writes arrays into a state, leaving what is not given and the padding of the
+ * last record as it was.  Packing converts: a master of DT_F32, DT_BF16 or DT_F24 as
+ * adambridge_convert_plane does, moments of DT_F32, DT_BF16 or DT_FP8 as adambridge_convert does; the
+ * layout's own type is copied bit for bit.  One pass over the state, on the calling thread's stream
+ * (asynchronous).  Each array is aligned to its values; at 16 bytes its accesses are wider.  Returns
+ * 0, ADAMBRIDGE_EBADN (n < 0), _EPDTYPE (no interleaved layout, or a master type it does not take),
+ * _EMVDTYPE (a moment type, or a second moment the layout has not), _ENULL, _ESCALES, _EALIGN or
+ * _EHIP. */
+ADAMBRIDGE_API int adambridge_unpack_state(const adambridge_state* state, const adambridge_arrays* to);
+ADAMBRIDGE_API int adambridge_pack_state(const adambridge_state* state, const adambridge_arrays* from);
+
 /* Summed cross-entropy of a slice of logits and its gradient (reference adambridge/losses.py:27-70),
  * on the calling thread's stream (asynchronous).  logits: rows x vocab values, contiguous
  * (ADAMBRIDGE_DT_F32 or _BF16); target: one class per row, a row whose target equals ignore_index
