@@ -76,14 +76,15 @@ struct DevSeg {
     int64_t n_main;      // [0, n_main) take the fused form, [n_main, n) the scalar-tail form
     int64_t tile_begin;  // first tile of this segment in the launch
     uint32_t idx0;       // uint32(offset): element i draws rounding bits at idx0 + i
-    uint32_t flags;      // kVec: every pointer allows 16-byte access; kSR: stochastic rounding;
+    uint32_t flags;      // kVec: every pointer allows the kernel's vector access (kVec4: that of four
+                         // elements, k_update); kSR: stochastic rounding;
                          // kPrev: out receives the weight of the master before the update;
                          // kFastDiv: the coefficients allow quot_fast (adamw8_fused)
     Coef c;
     uint32_t seed_m, seed_v, seed_p, pad;
 };
 static_assert(sizeof(DevSeg) == 144, "DevSeg layout");
-constexpr uint32_t kVec = 1u, kSR = 2u, kPrev = 4u, kFastDiv = 8u;
+constexpr uint32_t kVec = 1u, kSR = 2u, kPrev = 4u, kFastDiv = 8u, kVec4 = 16u;
 
 struct Launch {
     const DevSeg* table;     // device table when nsegs > kInline
@@ -339,9 +340,7 @@ __device__ __forceinline__ void store_out8(void* p, const float (&x)[8])
 
 // ------------------------------------------------ two elements per lane
 //
-// The FP32/BF16-moment kernel gives each lane two consecutive elements: one
-// small access per buffer per lane.  Measured on MI355X this streams faster
-// than wider per-lane chunks (fewer bytes in flight per lane to distinct rows).
+// Buffers whose alignment allows no wider access than two elements (k_update), and the pair layout.
 
 template <int DT>
 __device__ __forceinline__ void load2(const void* base, int64_t i, float& x0, float& x1)
@@ -414,6 +413,84 @@ __device__ __forceinline__ void store_out2(void* base, int64_t i, float x0, floa
     else if constexpr (OT == DT_F32) store2_f32(base, i, x0, x1);
 }
 
+// ------------------------------------------------ four elements per lane
+
+template <int DT>
+__device__ __forceinline__ void load4(const void* base, int64_t i, float (&x)[4])
+{
+    if constexpr (DT == DT_BF16) {
+        const u32x2 w = ld(reinterpret_cast<const u32x2*>(static_cast<const uint16_t*>(base) + i));
+        x[0] = bitsf(w.x << 16);
+        x[1] = bitsf(w.x & 0xffff0000u);
+        x[2] = bitsf(w.y << 16);
+        x[3] = bitsf(w.y & 0xffff0000u);
+    } else {
+        const f32x4 w = ld(reinterpret_cast<const f32x4*>(static_cast<const float*>(base) + i));
+        x[0] = w.x; x[1] = w.y; x[2] = w.z; x[3] = w.w;
+    }
+}
+
+__device__ __forceinline__ void store4_f32(void* base, int64_t i, const float (&x)[4])
+{
+    st(reinterpret_cast<f32x4*>(static_cast<float*>(base) + i), f32x4{x[0], x[1], x[2], x[3]});
+}
+
+template <int PT>
+__device__ __forceinline__ void load_master4(const DevSeg& s, int64_t i, float (&x)[4])
+{
+    if constexpr (PT == DT_F24) {
+        const u32x2 h = ld(reinterpret_cast<const u32x2*>(static_cast<const uint16_t*>(s.p) + i));
+        const uint32_t l = ld(reinterpret_cast<const uint32_t*>(s.p_lo + i));
+        x[0] = bitsf((h.x << 16) | ((l & 0xffu) << 8));
+        x[1] = bitsf((h.x & 0xffff0000u) | (l & 0xff00u));
+        x[2] = bitsf((h.y << 16) | ((l >> 8) & 0xff00u));
+        x[3] = bitsf((h.y & 0xffff0000u) | ((l >> 16) & 0xff00u));
+    } else {
+        load4<DT_F32>(s.p, i, x);
+    }
+}
+
+// Rounds and stores four new master values; x becomes the values stored.
+template <int PT, bool SR>
+__device__ __forceinline__ void store_master4(const DevSeg& s, int64_t i, float (&x)[4], uint32_t idx)
+{
+    if constexpr (PT == DT_F24) {
+        uint32_t b[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            b[k] = f24_round<SR>(x[k], SR ? hash32((idx + k) ^ s.seed_p) : 0u);
+            x[k] = bitsf(b[k]);
+        }
+        st(reinterpret_cast<u32x2*>(static_cast<uint16_t*>(s.p) + i),
+           u32x2{(b[0] >> 16) | (b[1] & 0xffff0000u), (b[2] >> 16) | (b[3] & 0xffff0000u)});
+        st(reinterpret_cast<uint32_t*>(s.p_lo + i), ((b[0] >> 8) & 0xffu) | (b[1] & 0xff00u) |
+                                                        ((b[2] & 0xff00u) << 8) | ((b[3] & 0xff00u) << 16));
+    } else {
+        store4_f32(s.p, i, x);
+    }
+}
+
+template <int MV, bool SR>
+__device__ __forceinline__ void store_moment4(void* base, int64_t i, const float (&x)[4], uint32_t idx, uint32_t seed)
+{
+    if constexpr (MV == DT_BF16) {
+        uint32_t h[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) h[k] = bf16_store<SR>(x[k], SR ? hash32((idx + k) ^ seed) : 0u);
+        st(reinterpret_cast<u32x2*>(static_cast<uint16_t*>(base) + i), u32x2{h[0] | (h[1] << 16), h[2] | (h[3] << 16)});
+    } else {
+        store4_f32(base, i, x);
+    }
+}
+
+template <int OT>
+__device__ __forceinline__ void store_out4(void* base, int64_t i, const float (&x)[4])
+{
+    if constexpr (OT == DT_BF16)
+        st(reinterpret_cast<u32x2*>(static_cast<uint16_t*>(base) + i), u32x2{bf16x2_rne(x[0], x[1]), bf16x2_rne(x[2], x[3])});
+    else if constexpr (OT == DT_F32) store4_f32(base, i, x);
+}
+
 // ------------------------------------------------------------ scalar access
 
 template <int DT>
@@ -483,6 +560,12 @@ __device__ __forceinline__ void store_out1(void* base, int64_t i, float x)
 // ALGO: AdamW or Lion; MV: moment storage (F32 / BF16); PT: master (F32 / F24);
 // GT: gradient (F32 / BF16); OT: working-weight output (NONE / F32 / BF16);
 // SR: stochastic rounding of BF16 moments and an FP24 master.
+//
+// Bound by HBM: five to seven streams, each array of its own.  Four elements a lane (16-byte FP32
+// accesses) where every pointer allows it, two elsewhere, one for what is left.  Alone the wider
+// lanes give 1-3% (0.5B list: FP24 master with a BF16 Lion moment 1253 -> 1215 us, with AdamW's 1619
+// -> 1598; others within 1%); with AdamW's FP32 moments what helps is fewer of them in flight
+// (launch_lds): 2438 -> 2335 us, 5.67 -> 5.93 TB/s.
 template <int ALGO, int MV, int PT, int GT, int OT, bool SR>
 __device__ __forceinline__ void update_tile(const DevSeg& s, int64_t tile, int64_t T)
 {
@@ -490,13 +573,37 @@ __device__ __forceinline__ void update_tile(const DevSeg& s, int64_t tile, int64
     const int64_t lo = (tile - s.tile_begin) * T;
     const int64_t hi = lo + T < n ? lo + T : n;
     const Coef c = s.c;
-    const int64_t nvec = (s.flags & kVec) ? (n_main & ~(int64_t)1) : 0;
     const bool prev = (s.flags & kPrev) != 0;   // uniform: out from the master as loaded
+    const int64_t nvec = (s.flags & kVec) ? (n_main & ~(int64_t)1) : 0;
+    const int64_t nquad = (s.flags & kVec4) ? (n_main & ~(int64_t)3) : 0;
+    int64_t qend = hi < nquad ? hi : nquad;
+    if (qend < lo) qend = lo;
     int64_t vend = hi < nvec ? hi : nvec;
-    if (vend < lo) vend = lo;
+    if (vend < qend) vend = qend;
 
-    // each workgroup streams one contiguous tile: pairs of elements, both in the fused range
-    for (int64_t i = lo + threadIdx.x * 2; i < vend; i += kThreads * 2) {
+    // each workgroup streams one contiguous tile: four elements a lane, all in the fused range
+    for (int64_t i = lo + threadIdx.x * 4; i < qend; i += kThreads * 4) {
+        const uint32_t idx = s.idx0 + (uint32_t)i;
+        float g[4], m[4], v[4] = {0.0f, 0.0f, 0.0f, 0.0f}, p[4];
+        load4<GT>(s.g, i, g);
+        load4<MV>(s.m, i, m);
+        if constexpr (ALGO == ALGO_ADAMW) load4<MV>(s.v, i, v);
+        load_master4<PT>(s, i, p);
+        if (prev) store_out4<OT>(s.out, i, p);
+        if constexpr (ALGO == ALGO_ADAMW) {
+            adamw_pair_fused(p[0], p[1], g[0], g[1], m[0], m[1], v[0], v[1], c);
+            adamw_pair_fused(p[2], p[3], g[2], g[3], m[2], m[3], v[2], v[3], c);
+        } else {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) p[k] = lion(p[k], g[k], m[k], c);
+        }
+        store_master4<PT, SR>(s, i, p, idx);
+        store_moment4<MV, SR>(s.m, i, m, idx, s.seed_m);
+        if constexpr (ALGO == ALGO_ADAMW) store_moment4<MV, SR>(s.v, i, v, idx, s.seed_v);
+        if (!prev) store_out4<OT>(s.out, i, p);
+    }
+    // pairs, both in the fused range: buffers without 4-element alignment, a last pair
+    for (int64_t i = qend + threadIdx.x * 2; i < vend; i += kThreads * 2) {
         const uint32_t idx = s.idx0 + (uint32_t)i;
         float g0, g1, m0, m1, v0 = 0.0f, v1 = 0.0f, p0, p1;
         load2<GT>(s.g, i, g0, g1);
@@ -1819,16 +1926,26 @@ inline bool kernel_is_fp8(int index)
 // 5: 3.11, 8: 3.12.  The
 // BF16 pairs lose with fewer workgroups (the 0.5B list: 1.76 against 1.67 ms with 6), and the
 // FP24-master FP8 kernels keep 8 (records, the 7B list: 8 per CU 16.28-16.66, 7: 16.18-16.55, 6:
-// 16.44-16.65, 5: 17.56-17.91).  Those run at the speed of their accesses alone: a form that makes
+// 16.44-16.65, 5: 17.56-17.91).  The separate arrays of FP32 / BF16 moments (k_update at 4 elements a
+// lane, the 0.5B list, us, 8 / 6 / 5 / 4 per CU): AdamW with FP32 moments 2448 / 2380 / 2335 / 2331
+// over an FP32 master (the 1.5B list 7574 / 7387 / 7240 / 7264), 2334 / 2272 / 2236 / 2234 over an
+// FP24 one -- held to 5, or 6 where the tile is 512 elements, two of the workgroup's wavefronts (19M
+// elements: 110 / 106 / 111 / 110); FP32 masters with AdamW's BF16 moments 1701 / 1684 / 1799 / 1798,
+// Lion's FP32 1660 / 1624 / 1746 / 1743 and BF16 1305 / 1304 / 1571 / 1571 -- held to 6; FP24 masters
+// with Lion's BF16 moment 1215 / 1259 / 1511 / 1511 -- kept at 8.
+// The FP24-master FP8 kernels run at the speed of their accesses alone: a form that makes
 // the same loads and stores and no arithmetic took 16.45 ms at 8 per CU, and its time falls as the
 // CU holds fewer workgroups (15.46 at 5, 15.15 at 3) while the arithmetic needs the wavefronts.
-inline size_t launch_lds(int index)
+inline size_t launch_lds(int index, int64_t tile)
 {
     constexpr size_t kCap6 = 24 * 1024;   // 6 workgroups of 24 KiB in 160 KiB; 7 would need 168
     constexpr size_t kCap5 = 32 * 1024;   // 5 of 32 KiB; 6 would need 192
     if (index < kNumKernels) {
         const int pt = (index / 6) % 2, mv = (index / 12) % 3, algo = index / 36;
-        if (mv != 2) return 0;   // FP8 moments only
+        if (mv != 2) {
+            if (algo == ALGO_ADAMW && mv == 0) return tile > kPairQuantum ? kCap5 : kCap6;
+            return pt == 0 ? kCap6 : 0;
+        }
         if (algo == ALGO_ADAMW) return pt == 0 ? kCap6 : 0;
         return pt == 0 ? kCap5 : kCap6;   // Lion: FP32 / FP24 master
     }
