@@ -377,9 +377,14 @@ class HipKernels:
         into the arrays (adambridge_unpack_state).  The memory must stay alive until the stream has
         run it."""
         fn = self._lib.adambridge_pack_state if pack else self._lib.adambridge_unpack_state
-        with torch.cuda.device(device):
-            self._lib.adambridge_set_stream(torch.cuda.current_stream(device).cuda_stream)
+        current = torch._C._cuda_getDevice()
+        index = current if device.index is None else device.index
+        self._lib.adambridge_set_stream(torch._C._cuda_getCurrentRawStream(index))
+        if index == current:   # a model's states are moved one by one: no context to enter for each
             rc = fn(ctypes.byref(state), ctypes.byref(arrays))
+        else:
+            with torch.cuda.device(index):
+                rc = fn(ctypes.byref(state), ctypes.byref(arrays))
         self._check(rc, "adambridge_pack_state" if pack else "adambridge_unpack_state")
 
     # -- cross-entropy ---------------------------------------------------------
@@ -481,3 +486,19 @@ def load() -> HipKernels:
         if _loaded is None:
             _loaded = HipKernels()
         return _loaded
+
+
+_bind_module = None
+
+
+def bind():
+    """The host module _bind (csrc/abh_bind.cpp).  Raises RuntimeError if it is not built."""
+    global _bind_module
+    if _bind_module is None:
+        try:
+            from . import _bind
+        except ImportError as exc:
+            raise RuntimeError(f"adambridge_amd/_bind.so is not built or does not load ({exc}): "
+                               "run `python -m adambridge_amd.build` (or __graft_entry__.build())") from exc
+        _bind_module = _bind
+    return _bind_module

@@ -13,6 +13,7 @@ from __future__ import annotations
 import os
 import subprocess
 import sys
+import sysconfig
 import tempfile
 from pathlib import Path
 
@@ -20,6 +21,8 @@ PKG = Path(__file__).resolve().parent
 ROOT = PKG.parent
 SOURCES = [PKG / "csrc" / name for name in ("adambridge_hip.hip", "abh_state.hip", "abh_loss.hip")]
 LIB = PKG / "libadambridge_hip.so"
+BIND_SOURCE = PKG / "csrc" / "abh_bind.cpp"   # host code over torch's C++ tensors: the Python module _bind
+BIND = PKG / "_bind.so"
 ARCH = os.environ.get("ADAMBRIDGE_HIP_ARCH", "gfx950")
 
 
@@ -37,13 +40,25 @@ def flags() -> list[str]:
             f"-I{ROOT / 'include'}"]
 
 
+def bind_command(out: Path) -> list[str]:
+    import torch
+    from torch.utils import cpp_extension
+
+    lib = Path(torch.__file__).resolve().parent / "lib"
+    includes = [f"-I{d}" for d in (ROOT / "include", *cpp_extension.include_paths(), sysconfig.get_paths()["include"])]
+    return ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-fvisibility=hidden",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *includes, str(BIND_SOURCE),
+            "-o", str(out), f"-L{lib}", "-ltorch_python", "-ltorch_cpu", "-lc10"]
+
+
 def build(verbose: bool = False) -> Path:
-    """Compile the library (always; a stale library is never reused): the sources side by side, then
-    one link."""
+    """Compile the library and the host module (always; a stale one is never reused): the sources side by
+    side, then one link."""
     with tempfile.TemporaryDirectory(prefix="adambridge_build_") as work:
         objects = [Path(work) / (src.stem + ".o") for src in SOURCES]
         compiles = [[hipcc(), *flags(), "-c", str(src), "-o", str(obj)] for src, obj in zip(SOURCES, objects)]
-        tmp = LIB.with_suffix(".so.tmp")
+        tmp, bind = LIB.with_suffix(".so.tmp"), BIND.with_suffix(".so.tmp")
+        compiles.append(bind_command(bind))
         link = [hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", *map(str, objects), "-o", str(tmp)]
         if verbose:
             print("\n".join(" ".join(cmd) for cmd in [*compiles, link]), file=sys.stderr)
@@ -56,8 +71,9 @@ def build(verbose: bool = False) -> Path:
             results.append((linked.stderr, linked.returncode))
         for output, code in results:
             if code != 0:
-                raise RuntimeError(f"hipcc failed ({code}):\n{output}")
+                raise RuntimeError(f"the compiler failed ({code}):\n{output}")
         os.replace(tmp, LIB)
+        os.replace(bind, BIND)
     return LIB
 
 

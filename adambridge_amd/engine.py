@@ -56,6 +56,7 @@ from .state import ParamState, arena_memory, choose_layout, new_states
 
 __all__ = ["UpdateEngine", "ParamSlot", "SmallGroup", "StepStats"]
 
+_SEGMENT_POINTER = ctypes.POINTER(_hip.Segment)
 _GRAD_CODES = {torch.bfloat16: _hip.DT_BF16, torch.float32: _hip.DT_F32}
 
 
@@ -63,7 +64,7 @@ class ParamSlot:
     """One parameter: its index (rounding stream), group, step count, state and kernel descriptor."""
 
     __slots__ = ("index", "param", "group", "numel", "step", "state", "out", "out_view", "submitted", "seg",
-                 "seg_ptr", "bound", "_small", "done_ev", "seg_group", "seg_out")
+                 "seg_ptr", "seg_addr", "bound", "plain", "in_place", "_small", "done_ev")
 
     def __init__(self, index: int, param: torch.Tensor, group: dict):
         self.index = index
@@ -77,11 +78,12 @@ class ParamSlot:
         self.submitted = False                      # updated (or queued) in the current step
         self.seg = _hip.Segment(n=self.numel, index=index)
         self.seg_ptr = ctypes.pointer(self.seg)
+        self.seg_addr = ctypes.addressof(self.seg)
         self.bound: ParamState | None = None        # the state whose buffers seg points at
+        self.plain = False                          # bound for good: the state's buffers do not alternate
+        self.in_place = False                       # the master is the parameter (no weight to write)
         self._small: weakref.ref | None = None
         self.done_ev: torch.cuda.Event | None = None   # recorded after the slot's latest update
-        self.seg_group: _hip.Group | None = None    # the group struct seg points at
-        self.seg_out: tuple | None = None           # (out, out_dtype, reserved) seg holds
 
     @property
     def initialized(self) -> bool:
@@ -159,6 +161,10 @@ class _Hyper:
                         float(group["weight_decay"]), self.seed, self.stochastic, 0)
         return struct
 
+    def address(self, group: dict) -> int:
+        """The address of the group's struct, refreshed."""
+        return ctypes.addressof(self.refresh(group))
+
 
 class _Lanes:
     """A device's two streams besides the caller's, for ``update_stream="side"``: updates run on
@@ -199,6 +205,7 @@ class UpdateEngine:
         if master_precision not in _hip.MASTER_CODES:
             raise ValueError(f"master_precision must be one of {sorted(_hip.MASTER_CODES)}")
         self.kernels = _hip.load()
+        self._bind = _hip.bind()
         self.algorithm = algorithm
         self._algo_code = _hip.ALGORITHMS[algorithm]
         self.lion = algorithm == "lion"
@@ -309,6 +316,8 @@ class UpdateEngine:
         slot.state = state
         state.bind(slot.seg)
         slot.bound = state
+        slot.plain = not state.alternates
+        slot.in_place = state.master_is_param
 
     def rebuild(self, slots: list[ParamSlot], precision: str | None = None, masters: list | None = None,
                 moments: list[dict[str, MomentStore] | None] | None = None) -> None:
@@ -418,19 +427,53 @@ class UpdateEngine:
             # a delayed first update owes the parameter nothing: its weight is the one the master was
             # made from (which an FP24 master holds only rounded)
             out, dtype, buffered = None, None, False
-        # fields that rarely change are written only when they do (host time per step with ~300 slots)
-        want = (out, _hip.DT_NONE if out is None else _hip.DT_F32 if dtype is torch.float32 else _hip.DT_BF16,
-                _hip.SEG_OUT_PREVIOUS if self.delay and out is not None else 0)
-        if slot.seg_out != want:
-            seg.out, seg.out_dtype, seg.reserved = want
-            slot.seg_out = want
+        seg.out = out
+        seg.out_dtype = _hip.DT_NONE if out is None else _hip.DT_F32 if dtype is torch.float32 else _hip.DT_BF16
+        seg.reserved = _hip.SEG_OUT_PREVIOUS if self.delay and out is not None else 0
         seg.step = slot.step
-        if slot.seg_group is not group:
-            seg.group = ctypes.pointer(group)
-            slot.seg_group = group
+        seg.group = ctypes.pointer(group)
         return slot.seg_ptr, buffered
 
     # ------------------------------------------------------------ submission
+
+    def update_plain(self, slots: list[ParamSlot], grads: list[torch.Tensor], hooked: bool = False) -> bool:
+        """:meth:`update` for the ordinary case -- every slot with its state, on one device, contiguous
+        tensors, weights written in place, on the current stream, untimed -- its per-tensor work done
+        natively (_bind.describe).  False, with nothing changed, if it is not that case (or a slot was
+        updated in this step already)."""
+        if self.apart or self.timing or self.launch_log is not None or not slots \
+                or (hooked and not self.overlap_writeback and not self.delay):
+            return False
+        device = slots[0].param.device
+        index = device.index
+        if device.type != "cuda" or slots[0].state is None:   # (the first update builds the states)
+            return False
+        array = (_SEGMENT_POINTER * len(slots))()
+        if not self._bind.describe(slots, grads, array, index, self._algo_code, self.delay, self._hyper.address):
+            return False
+        stream_id, handle = torch._C._cuda_getCurrentStream(index)[0], torch._C._cuda_getCurrentRawStream(index)
+        try:
+            self.kernels.set_stream(handle)
+            if torch._C._cuda_getDevice() == index:
+                self.kernels.multi_step(None, array)
+            else:
+                with torch.cuda.device(device):
+                    self.kernels.multi_step(None, array)
+        except BaseException:
+            for slot in slots:   # nothing was enqueued: the library validates and plans before launching
+                slot.step -= 1
+            raise
+        self._bind.record(grads, stream_id, index)   # the gradients are released after this
+        with self._lock:
+            if self.delay:
+                for slot in slots:
+                    self._owed.pop(slot, None)
+                    self._fresh[slot] = None
+            held = self._streams.get(device)
+            if held is None or handle not in held:
+                self._note(device, torch.cuda.current_stream(device))
+            self._num_updates += len(slots)
+        return True
 
     def update(self, slots: list[ParamSlot], grads: list[torch.Tensor], hooked: bool = False) -> None:
         """Enqueue one fused update of ``slots`` with ``grads``, one launch per device, on the device's side
@@ -523,6 +566,8 @@ class UpdateEngine:
         with self._lock:
             streams = {d: dict(ss) for d, ss in self._streams.items()}
         for device, members in streams.items():
+            if len(members) == 1 and torch._C._cuda_getCurrentRawStream(device.index) in members:
+                continue   # nothing on any other stream
             current = torch.cuda.current_stream(device)
             for key, s in members.items():
                 if key != current.cuda_stream:

@@ -43,6 +43,7 @@ import torch
 import torch._dynamo  # noqa: F401 -- imported here, not by the first torch.compiler.disable() call: that import
 #                       keeps the frames on the stack alive, which would pin the optimizer being built
 
+from . import _hip
 from .engine import ParamSlot, SmallGroup, StepStats, UpdateEngine
 from .precision import (FP32Store, _checked, bytes_per_param, canonical_master_precision, canonical_precision,
                         check_master_state, make_store, store_from_state_dict)
@@ -120,10 +121,9 @@ class _Registry:
                 per_device.setdefault(p.device, []).append(slot)
         self.small += [SmallGroup(members) for members in per_device.values()]
 
-    def pending(self, *, include_small: bool = True) -> list[ParamSlot]:
-        """Slots with a gradient and no update yet in this step."""
-        return [s for s in self.ordered if not s.submitted and s.param.grad is not None
-                and (include_small or s.small is None)]
+    def pending(self, *, include_small: bool = True) -> tuple[list[ParamSlot], list[torch.Tensor]]:
+        """Slots with a gradient and no update yet in this step, and their gradients."""
+        return _hip.bind().pending(self.ordered, include_small)
 
     def hook_targets(self, params: Iterable[torch.Tensor] | None = None) -> list[torch.Tensor]:
         """The parameters that get a gradient hook: those of ``params`` (default: every registered one)
@@ -132,8 +132,7 @@ class _Registry:
         return [s.param for s in slots if s.param.requires_grad and s.small is None]
 
     def new_step(self) -> None:
-        for slot in self.ordered:
-            slot.submitted = False
+        _hip.bind().mark(self.ordered, False)
 
 
 class _StepWindow:
@@ -526,14 +525,19 @@ class AdamBridge(torch.optim.Optimizer):
 
     def _submit(self, slots: list[ParamSlot], grads: list[torch.Tensor], hooked: bool, release: bool) -> None:
         """One launch for ``slots`` (optimizer.py:310-321, batched)."""
-        self._check_submission(slots, grads)
         try:
-            self._engine.update(slots, grads, hooked=hooked)
+            done = self._engine.update_plain(slots, grads, hooked=hooked)
         except Exception as exc:   # surfaced as the reference surfaces its workers' errors (engine.py:1150-1158)
             raise RuntimeError(f"adambridge update failed: {exc}") from exc
-        for slot in slots:
-            slot.submitted = True
-            if release:
+        if not done:
+            self._check_submission(slots, grads)
+            try:
+                self._engine.update(slots, grads, hooked=hooked)
+            except Exception as exc:
+                raise RuntimeError(f"adambridge update failed: {exc}") from exc
+        _hip.bind().mark(slots, True)
+        if release:
+            for slot in slots:
                 slot.param.grad = None
 
     def step_sync(self) -> StepStats:
@@ -555,14 +559,14 @@ class AdamBridge(torch.optim.Optimizer):
         """What the hooks did not update: with gradient accumulation, the parameters whose window the
         step cut short; the small parameters, one launch per device."""
         if self.accumulation_steps > 1:
-            late = self._registry.pending(include_small=False)
+            late, grads = self._registry.pending(include_small=False)
             if late:
-                self._submit(late, [s.param.grad for s in late], hooked=False, release=False)
+                self._submit(late, grads, hooked=False, release=False)
         release = self.release_grads and self._hooks.active
         for batch in self._registry.small:
-            live = [s for s in batch.slots if not s.submitted and s.param.grad is not None]
+            live, grads = _hip.bind().pending(batch.slots, True)
             if live:
-                self._submit(live, [s.param.grad for s in live], hooked=self._hooks.active, release=release)
+                self._submit(live, grads, hooked=self._hooks.active, release=release)
 
     def flush(self) -> None:
         """Apply every pending (delayed) update to the parameters (optimizer.py:432-436)."""
@@ -578,9 +582,9 @@ class AdamBridge(torch.optim.Optimizer):
         if closure is not None:
             with torch.enable_grad():
                 loss = closure()
-        todo = self._registry.pending()
+        todo, grads = self._registry.pending()
         if todo:
-            self._submit(todo, [s.param.grad for s in todo], hooked=False, release=False)
+            self._submit(todo, grads, hooked=False, release=False)
         self.step_sync()
         return loss
 

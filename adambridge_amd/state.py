@@ -367,7 +367,9 @@ class _Interleaved(ParamState):
             if role in moments:
                 store = _kernel_store(moments[role], role, self.device)
                 by_format.setdefault(store.precision, {})[role] = store
-        for precision, stores in by_format.items() or [("fp32", {})]:
+        if not by_format:
+            self._move(arrays, pack=True)
+        for precision, stores in by_format.items():
             arrays.mv_dtype = _hip.MOMENT_CODES[precision]
             for role, store in stores.items():
                 values, scale = store.native_buffers
