@@ -410,11 +410,13 @@ class HipKernels:
         return loss, stats
 
     def cross_entropy_backward(self, logits: torch.Tensor, target: torch.Tensor, ignore_index: int,
-                               stats: torch.Tensor, gout: torch.Tensor) -> torch.Tensor:
+                               stats: torch.Tensor, gout: torch.Tensor, out: torch.Tensor | None = None
+                               ) -> torch.Tensor:
         """The gradient of :meth:`cross_entropy`'s sum with respect to the logits, times ``gout`` (an FP32
-        scalar on the device), in the logits' type (adambridge_cross_entropy_backward)."""
+        scalar on the device), in the logits' type (adambridge_cross_entropy_backward): a new tensor,
+        or ``out``, which may be the logits themselves."""
         rows, vocab = logits.shape
-        grad = torch.empty_like(logits)
+        grad = torch.empty_like(logits) if out is None else out
         with torch.cuda.device(logits.device):
             self._lib.adambridge_set_stream(torch.cuda.current_stream(logits.device).cuda_stream)
             rc = self._lib.adambridge_cross_entropy_backward(

@@ -29,21 +29,45 @@ __all__ = ["causal_lm_loss"]
 _MAX_ROWS = 1 << 23   # adambridge_cross_entropy's
 
 
-def _kernels_apply(logits: torch.Tensor, target: torch.Tensor) -> bool:
-    """Whether the library's cross-entropy takes this slice: plain contiguous tensors of its types on one
-    GPU, and nothing that needs the torch operations themselves -- a trace or compilation, a function
+def _observed() -> bool:
+    """Whether something needs the torch operations themselves: a trace or compilation, a function
     transform (vmap, functorch grad), forward-mode derivatives, a mode that observes operations."""
-    if (torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._are_functorch_transforms_active()
-            or forward_ad._current_level >= 0 or torch._C._len_torch_dispatch_stack()
-            or torch._C._len_torch_function_stack()):
-        return False
-    return (type(logits) is torch.Tensor and type(target) is torch.Tensor
-            and logits.is_cuda and target.device == logits.device
-            and logits.dtype in (torch.bfloat16, torch.float32) and target.dtype == torch.int64
-            and logits.dim() == 2 and target.dim() == 1 and target.numel() == logits.shape[0]
-            and logits.is_contiguous() and target.is_contiguous() and not logits.is_neg()
-            and 0 < logits.shape[0] <= _MAX_ROWS and logits.shape[1] > 0
+    return bool(torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._are_functorch_transforms_active()
+                or forward_ad._current_level >= 0 or torch._C._len_torch_dispatch_stack()
+                or torch._C._len_torch_function_stack())
+
+
+def _ordinary(values: torch.Tensor, target: torch.Tensor) -> bool:
+    """Whether rows of ``values`` and their ``target`` are plain contiguous tensors of the kernels' types on
+    one GPU."""
+    return (type(target) is torch.Tensor and values.is_cuda and target.device == values.device
+            and values.dtype in (torch.bfloat16, torch.float32) and target.dtype == torch.int64
+            and values.dim() == 2 and target.dim() == 1 and target.numel() == values.shape[0]
+            and values.is_contiguous() and target.is_contiguous() and not values.is_neg()
+            and 0 < values.shape[0] <= _MAX_ROWS and values.shape[1] > 0)
+
+
+def _kernels_apply(logits: torch.Tensor, target: torch.Tensor) -> bool:
+    """Whether the library's cross-entropy takes this slice."""
+    return (not _observed() and type(logits) is torch.Tensor and _ordinary(logits, target)
             and logits.data_ptr() % 16 == 0)   # so that the gradient, a new tensor, shares its alignment
+
+
+def _head_applies(head, h: torch.Tensor, targets: torch.Tensor) -> bool:
+    """Whether ``head(h)`` is exactly ``h @ head.weight.T`` on plain tensors, so that :class:`_HeadLoss` may
+    take the products itself: a torch.nn.Linear without a bias, with nothing hooked, replaced or cast
+    around its call."""
+    if type(head) is not torch.nn.Linear or head.bias is not None or "forward" in head.__dict__ or _observed():
+        return False
+    hooks = torch.nn.modules.module
+    if (head._forward_hooks or head._forward_pre_hooks or head._backward_hooks or head._backward_pre_hooks
+            or hooks._global_forward_hooks or hooks._global_forward_pre_hooks or hooks._global_backward_hooks
+            or hooks._global_backward_pre_hooks or torch.is_autocast_enabled("cuda")):
+        return False
+    w = head.weight
+    return (type(h) in (torch.Tensor, torch.nn.Parameter) and type(w) in (torch.Tensor, torch.nn.Parameter)
+            and _ordinary(h, targets) and w.device == h.device and w.dtype == h.dtype and w.dim() == 2
+            and w.is_contiguous() and not w.is_neg() and w.shape[1] == h.shape[1] and w.shape[0] > 0)
 
 
 class _SliceLoss(torch.autograd.Function):
@@ -64,6 +88,51 @@ class _SliceLoss(torch.autograd.Function):
             loss = _torch_loss_sum(logits, target, ctx.ignore_index)
             return torch.autograd.grad(loss, logits, gout, create_graph=True)[0], None, None
         return _hip.load().cross_entropy_backward(logits, target, ctx.ignore_index, stats, gout), None, None
+
+
+class _HeadLoss(torch.autograd.Function):
+    """Summed cross-entropy of ``h @ weight.T``, ``chunk`` rows at a time.  The backward pass computes each
+    slice's logits again, as the checkpointed slices do, but neither their statistics (two floats per
+    row, kept) nor a gradient beside them (it takes the logits' place), and the weight's gradient is
+    added up inside the products (rounded once per slice, where the slices' gradients were each
+    rounded, then added and rounded)."""
+
+    @staticmethod
+    def forward(ctx, h, weight, targets, ignore_index, chunk):
+        k = _hip.load()
+        total, kept = h.new_zeros((), dtype=torch.float32), []
+        for h_part, t_part in zip(torch.split(h, chunk), torch.split(targets, chunk)):
+            loss, stats = k.cross_entropy(torch.mm(h_part, weight.t()), t_part, ignore_index)
+            total += loss
+            kept.append(stats)
+        ctx.save_for_backward(h, weight, targets, *kept)
+        ctx.ignore_index, ctx.chunk = ignore_index, chunk
+        return total
+
+    @staticmethod
+    def backward(ctx, gout):
+        h, weight, targets, *kept = ctx.saved_tensors
+        wanted = ctx.needs_input_grad[:2]
+        if torch.is_grad_enabled():   # create_graph: gradients that are differentiated in turn
+            total = sum(_torch_loss_sum(torch.mm(a, weight.t()), t, ctx.ignore_index)
+                        for a, t in zip(torch.split(h, ctx.chunk), torch.split(targets, ctx.chunk)))
+            inputs = [x for x, want in zip((h, weight), wanted) if want]
+            grads = iter(torch.autograd.grad(total, inputs, gout, create_graph=True))
+            return (*(next(grads) if want else None for want in wanted), None, None, None)
+        k = _hip.load()
+        dh = torch.empty_like(h) if wanted[0] else None
+        dw = None
+        parts = zip(torch.split(h, ctx.chunk), torch.split(targets, ctx.chunk), kept,
+                    torch.split(h if dh is None else dh, ctx.chunk))
+        for h_part, t_part, stats, dh_part in parts:
+            logits = torch.mm(h_part, weight.t())
+            grad = k.cross_entropy_backward(logits, t_part, ctx.ignore_index, stats, gout, out=logits)
+            if wanted[0]:
+                torch.mm(grad, weight, out=dh_part)
+            if wanted[1]:
+                dw = torch.mm(grad.t(), h_part) if dw is None else dw.addmm_(grad.t(), h_part)
+            del logits, grad
+        return dh, dw, None, None, None
 
 
 def _torch_loss_sum(logits: torch.Tensor, target: torch.Tensor, ignore_index: int) -> torch.Tensor:
@@ -91,7 +160,8 @@ def causal_lm_loss(hidden_states: torch.Tensor, lm_head: Callable[[torch.Tensor]
     no target); the mean runs over positions whose target is not ``ignore_index`` -- the Hugging
     Face causal-LM loss.  ``hidden_states``: ``[batch, seq, hidden]``; ``lm_head``: a module or
     function mapping ``[n, hidden]`` to ``[n, vocab]``; ``labels``: ``[batch, seq]`` token ids.
-    With gradients enabled, each slice runs under non-reentrant ``torch.utils.checkpoint``.
+    With gradients enabled, each slice runs under non-reentrant ``torch.utils.checkpoint``, or (a
+    plain ``torch.nn.Linear`` head on the GPU) in one function of the same memory (:class:`_HeadLoss`).
     """
     if hidden_states.dim() != 3:
         raise ValueError(f"hidden_states must be [batch, seq, hidden], got shape {tuple(hidden_states.shape)}")
@@ -106,6 +176,8 @@ def causal_lm_loss(hidden_states: torch.Tensor, lm_head: Callable[[torch.Tensor]
     targets[:, :-1] = labels[:, 1:]
     targets = targets.reshape(-1).to(h.device)
     n_scored = (targets != ignore_index).sum()
+    if torch.is_grad_enabled() and _head_applies(lm_head, h, targets) and (h.requires_grad or lm_head.weight.requires_grad):
+        return _HeadLoss.apply(h, lm_head.weight, targets, ignore_index, chunk_tokens) / n_scored.clamp(min=1)
     recompute = torch.is_grad_enabled() and h.requires_grad
     total = h.new_zeros((), dtype=torch.float32)
     for h_part, t_part in zip(torch.split(h, chunk_tokens), torch.split(targets, chunk_tokens)):

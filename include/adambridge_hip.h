@@ -478,7 +478,7 @@ ADAMBRIDGE_API int adambridge_pack_state(const adambridge_state* state, const ad
  * the gradient, two floats per row to stats (the row's maximum and the reciprocal of its sum of
  * exponentials); work holds adambridge_cross_entropy_work(rows, vocab) bytes of scratch, 8-byte
  * aligned.  adambridge_cross_entropy_backward writes (softmax - one_hot(target)) * gout[0] to grad, in
- * the logits' type.  All of it is computed in FP32; sums are taken in a fixed order.  A target
+ * the logits' type; grad may be logits.  All of it is computed in FP32; sums are taken in a fixed order.  A target
  * outside [0, vocab) other than ignore_index makes the loss NaN (nothing is read for it).  Returns 0,
  * ADAMBRIDGE_EBADN (rows outside 1 .. 2^23, vocab < 1), _EMVDTYPE, _ENULL, _EALIGN (grad at another offset
  * from a 16-byte boundary than logits) or _EHIP; adambridge_cross_entropy_work the bytes, or

@@ -102,17 +102,20 @@ def test_causal_lm_loss_takes_the_kernels_and_agrees_with_torch(dtype, monkeypat
     calls = []
     k = _hip.load()
     real = k.cross_entropy_backward
-    monkeypatch.setattr(k, "cross_entropy_backward", lambda *a: calls.append(1) or real(*a))
+    monkeypatch.setattr(k, "cross_entropy_backward", lambda *a, **kw: calls.append(kw) or real(*a, **kw))
     got = _grads(*problem)
-    assert len(calls) == 3   # 80 positions, 32 at a time
+    assert len(calls) == 3 and all("out" in kw for kw in calls)   # 80 positions, 32 at a time, a plain head
     with torch.autograd.graph.save_on_cpu():
         moved = _grads(*problem)
+    monkeypatch.setattr(losses, "_head_applies", lambda *a: False)
+    sliced = _grads(*problem)
+    assert len(calls) == 9 and not calls[-1]
     monkeypatch.setattr(losses, "_kernels_apply", lambda *a: False)
     want = _grads(*problem)
     # two roundings of the logits' gradient to BF16 (2^-8 apart at most, at random) before the products
     tol = 2.0 ** -8 if dtype == torch.bfloat16 else 1e-5
-    for a, b, c in zip(got, want, moved):
-        assert (a - b).norm() <= tol * b.norm() and torch.equal(a, c)
+    for a, b, c, d in zip(got, want, moved, sliced):
+        assert (a - b).norm() <= tol * b.norm() and (d - b).norm() <= tol * b.norm() and torch.equal(a, c)
 
 
 def test_second_derivatives_and_transforms_use_torch_operations(monkeypatch):
@@ -149,3 +152,55 @@ def test_other_types_and_strides_use_torch_operations():
     assert not losses._kernels_apply(base.cpu(), target.cpu())
     loss = losses._slice_loss_sum(base.half(), target, lambda x: x, IGNORE)
     assert torch.allclose(loss, F.cross_entropy(base.half().float(), target, reduction="sum"))
+
+
+@pytest.mark.parametrize("frozen", ["none", "hidden", "weight"])
+def test_a_plain_head_matches_float64(frozen, monkeypatch):
+    """_HeadLoss's gradients, with either input frozen, a seed gradient and a second derivative."""
+    hidden, head, labels = _problem(torch.float32, vocab=301)
+    hidden.requires_grad_(frozen != "hidden")
+    head.weight.requires_grad_(frozen != "weight")
+    inputs = [x for x in (hidden, head.weight) if x.requires_grad]
+    assert losses._head_applies(head, hidden.reshape(80, 64), torch.zeros(80, dtype=torch.int64, device="cuda"))
+    loss = ab.causal_lm_loss(hidden, head, labels, chunk_tokens=32)
+    grads = torch.autograd.grad(loss, inputs, torch.tensor(0.3, device="cuda"))
+    h64, w64 = hidden.detach().double().requires_grad_(), head.weight.detach().double().requires_grad_()
+    target = torch.full_like(labels, IGNORE)
+    target[:, :-1] = labels[:, 1:]
+    want = F.cross_entropy((h64.reshape(80, 64) @ w64.T), target.reshape(-1), ignore_index=IGNORE)
+    exact = dict(zip(("hidden", "weight"), torch.autograd.grad(want, (h64, w64), torch.tensor(0.3, device="cuda").double())))
+    assert torch.allclose(loss.double(), want, rtol=1e-6)
+    for g, name in zip(grads, [n for n in ("hidden", "weight") if n != frozen]):
+        assert (g.double() - exact[name]).norm() <= 1e-5 * exact[name].norm()   # FP32 sums of 301 terms
+    loss = ab.causal_lm_loss(hidden, head, labels, chunk_tokens=32)
+    first = torch.autograd.grad(loss, inputs, create_graph=True)
+    second = torch.autograd.grad(sum(g.square().sum() for g in first), inputs)
+    monkeypatch.setattr(losses, "_head_applies", lambda *a: False)
+    monkeypatch.setattr(losses, "_kernels_apply", lambda *a: False)
+    loss = ab.causal_lm_loss(hidden, head, labels, chunk_tokens=80)
+    first = torch.autograd.grad(loss, inputs, create_graph=True)
+    for a, b in zip(second, torch.autograd.grad(sum(g.square().sum() for g in first), inputs)):
+        assert (a - b).norm() <= 1e-4 * b.norm()
+
+
+def test_heads_that_are_called_as_they_are():
+    """Anything but a bare Linear keeps its own call."""
+    hidden, head, labels = _problem(torch.bfloat16)
+    h, t = hidden.reshape(80, 64), torch.zeros(80, dtype=torch.int64, device="cuda")
+    assert losses._head_applies(head, h, t)
+    assert not losses._head_applies(lambda x: head(x), h, t)
+    assert not losses._head_applies(torch.nn.Linear(64, 9, device="cuda", dtype=torch.bfloat16), h, t)   # a bias
+    assert not losses._head_applies(head, h.float(), t) and not losses._head_applies(head, h[::2], t[::2])
+    assert not losses._head_applies(head.cpu(), h, t)
+    head.cuda()
+    handle = head.register_forward_hook(lambda *a: None)
+    assert not losses._head_applies(head, h, t)
+    handle.remove()
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert not losses._head_applies(head, h, t)
+    head.forward = lambda x: F.linear(x, head.weight)
+    assert not losses._head_applies(head, h, t)
+    del head.forward
+    assert losses._head_applies(head, h, t)
+    torch.nn.utils.parametrizations.weight_norm(head)
+    assert not losses._head_applies(head, h, t)
