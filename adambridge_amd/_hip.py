@@ -121,7 +121,7 @@ EXPORTS = (
     "adambridge_multi_step_noalloc", "adambridge_stream_copy", "adambridge_recycle_device_memory",
     "adambridge_convert_plane", "adambridge_capabilities", "adambridge_cross_entropy_work",
     "adambridge_cross_entropy", "adambridge_cross_entropy_backward", "adambridge_unpack_state",
-    "adambridge_pack_state",
+    "adambridge_pack_state", "adambridge_matmul_work", "adambridge_matmul",
 )
 
 
@@ -164,6 +164,8 @@ def open_library(path: Path = LIB_PATH) -> ctypes.CDLL:
         "adambridge_capabilities": (ctypes.c_uint32, []),
         "adambridge_unpack_state": (ctypes.c_int, [ctypes.POINTER(State), ctypes.POINTER(Arrays)]),
         "adambridge_pack_state": (ctypes.c_int, [ctypes.POINTER(State), ctypes.POINTER(Arrays)]),
+        "adambridge_matmul_work": (i64, [i64, i64, i64]),
+        "adambridge_matmul": (ctypes.c_int, [vp, vp, vp, i64, i64, i64, vp]),
         "adambridge_cross_entropy_work": (i64, [i64, i64]),
         "adambridge_cross_entropy": (ctypes.c_int, [vp, i32, vp, i64, i64, i64, vp, vp, vp]),
         "adambridge_cross_entropy_backward": (ctypes.c_int, [vp, i32, vp, i64, i64, i64, vp, vp, vp]),
@@ -424,6 +426,18 @@ class HipKernels:
                 stats.data_ptr(), gout.data_ptr(), grad.data_ptr())
         self._check(rc, "adambridge_cross_entropy_backward")
         return grad
+
+    def matmul(self, a: torch.Tensor, b: torch.Tensor, out: torch.Tensor) -> None:
+        """``out`` = ``a @ b`` for contiguous bfloat16 matrices on the current stream (adambridge_matmul)."""
+        (m, k), n = a.shape, b.shape[1]
+        nbytes = self._lib.adambridge_matmul_work(m, n, k)
+        if nbytes < 0:
+            self._check(nbytes, "adambridge_matmul_work")
+        work = torch.empty(nbytes // 4, dtype=torch.float32, device=a.device)
+        with torch.cuda.device(a.device):
+            self._lib.adambridge_set_stream(torch.cuda.current_stream(a.device).cuda_stream)
+            rc = self._lib.adambridge_matmul(a.data_ptr(), b.data_ptr(), out.data_ptr(), m, n, k, work.data_ptr())
+        self._check(rc, "adambridge_matmul")
 
     def fused_adamw(self, master: torch.Tensor, grad: torch.Tensor, m: torch.Tensor, v: torch.Tensor,
                     out: torch.Tensor | None, hp: HParams, lo: int, hi: int) -> None:

@@ -19,7 +19,7 @@ from pathlib import Path
 
 PKG = Path(__file__).resolve().parent
 ROOT = PKG.parent
-SOURCES = [PKG / "csrc" / name for name in ("adambridge_hip.hip", "abh_state.hip", "abh_loss.hip")]
+SOURCES = [PKG / "csrc" / name for name in ("adambridge_hip.hip", "abh_state.hip", "abh_loss.hip", "abh_gemm.hip")]
 LIB = PKG / "libadambridge_hip.so"
 BIND_SOURCE = PKG / "csrc" / "abh_bind.cpp"   # host code over torch's C++ tensors: the Python module _bind
 BIND = PKG / "_bind.so"

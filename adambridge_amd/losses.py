@@ -90,6 +90,17 @@ class _SliceLoss(torch.autograd.Function):
         return _hip.load().cross_entropy_backward(logits, target, ctx.ignore_index, stats, gout), None, None
 
 
+def _matmul_into(out: torch.Tensor, a: torch.Tensor, b: torch.Tensor) -> None:
+    """``out`` = ``a @ b``: by the library's split product (csrc/abh_gemm.hip) where the inner dimension is long
+    and the result small -- there the BLAS library leaves most of the chip idle -- else by torch."""
+    (m, k), n = a.shape, b.shape[1]
+    if (a.dtype == torch.bfloat16 and 1 << 14 <= k <= 1 << 22 and m * n <= 1 << 22 and n % 4 == 0 and k % 8 == 0
+            and a.data_ptr() % 16 == 0 and b.data_ptr() % 8 == 0 and out.data_ptr() % 8 == 0):
+        _hip.load().matmul(a, b, out)
+    else:
+        torch.mm(a, b, out=out)
+
+
 class _HeadLoss(torch.autograd.Function):
     """Summed cross-entropy of ``h @ weight.T``, ``chunk`` rows at a time.  The backward pass computes each
     slice's logits again, as the checkpointed slices do, but neither their statistics (two floats per
@@ -128,7 +139,7 @@ class _HeadLoss(torch.autograd.Function):
             logits = torch.mm(h_part, weight.t())
             grad = k.cross_entropy_backward(logits, t_part, ctx.ignore_index, stats, gout, out=logits)
             if wanted[0]:
-                torch.mm(grad, weight, out=dh_part)
+                _matmul_into(dh_part, grad, weight)
             if wanted[1]:
                 dw = torch.mm(grad.t(), h_part) if dw is None else dw.addmm_(grad.t(), h_part)
             del logits, grad

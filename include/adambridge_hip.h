@@ -471,6 +471,16 @@ typedef struct adambridge_arrays {
 ADAMBRIDGE_API int adambridge_unpack_state(const adambridge_state* state, const adambridge_arrays* to);
 ADAMBRIDGE_API int adambridge_pack_state(const adambridge_state* state, const adambridge_arrays* from);
 
+/* c = a b: a is m x k, b k x n, c m x n, all BF16, row-major and contiguous, summed in FP32 and rounded once,
+ * for a long k and a small result (the hidden states' gradient of a language-model head); the
+ * matrix cores' order of sums, the same for every call of the same sizes.  work holds
+ * adambridge_matmul_work(m, n, k) bytes, 16-byte aligned; a is 16-byte and b and c 8-byte aligned.
+ * On the calling thread's stream (asynchronous).  Returns 0, ADAMBRIDGE_EBADN (a size below 1 or above
+ * 2^22, n not a multiple of 4, k not of 8), _ENULL, _EALIGN or _EHIP; adambridge_matmul_work the bytes, or
+ * ADAMBRIDGE_EBADN. */
+ADAMBRIDGE_API int64_t adambridge_matmul_work(int64_t m, int64_t n, int64_t k);
+ADAMBRIDGE_API int adambridge_matmul(const void* a, const void* b, void* c, int64_t m, int64_t n, int64_t k, void* work);
+
 /* Summed cross-entropy of a slice of logits and its gradient (reference adambridge/losses.py:27-70),
  * on the calling thread's stream (asynchronous).  logits: rows x vocab values, contiguous
  * (ADAMBRIDGE_DT_F32 or _BF16); target: one class per row, a row whose target equals ignore_index

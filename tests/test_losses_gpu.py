@@ -204,3 +204,35 @@ def test_heads_that_are_called_as_they_are():
     assert losses._head_applies(head, h, t)
     torch.nn.utils.parametrizations.weight_norm(head)
     assert not losses._head_applies(head, h, t)
+
+
+# one row, the ends of a tile (256 x 128), a step (64 terms) and a split; rows and columns past a tile
+@pytest.mark.parametrize("m,n,k", [(1, 4, 8), (3, 8, 64), (33, 124, 72), (255, 128, 1024), (256, 132, 2056), (257, 4, 4096),
+                                   (1024, 896, 16392), (333, 1536, 50264), (2, 260, 151936)])
+def test_split_product_matches_float64(m, n, k):
+    gen = torch.Generator("cuda").manual_seed(m + n)
+    a = torch.randn(m, k, generator=gen, device="cuda").bfloat16()
+    b = torch.randn(k, n, generator=gen, device="cuda").bfloat16()
+    room = torch.full((m + 2, n), 7.0, dtype=torch.bfloat16, device="cuda")
+    _hip.load().matmul(a, b, room[1:m + 1])
+    want = a.double() @ b.double()
+    # one rounding to BF16 (8 significant bits: half a last place is at most 2^-8 of the value), and FP32
+    # sums of k products: each of the k additions off by 2^-24 of a partial sum, at most |a| |b| in all
+    bound = want.abs() * 2.0 ** -8 + (a.double().abs() @ b.double().abs()) * 2.0 ** -24 * k ** 0.5 + 1e-30
+    assert ((room[1:m + 1].double() - want).abs() <= bound).all()
+    assert (room[0] == 7).all() and (room[-1] == 7).all()
+
+
+def test_which_products_are_split(monkeypatch):
+    k = _hip.load()
+    calls = []
+    monkeypatch.setattr(k, "matmul", lambda a, b, out: calls.append(a.shape))
+    def try_(m, n, kk, dtype=torch.bfloat16, offset=0):
+        calls.clear()
+        a = torch.zeros(m * kk + offset, dtype=dtype, device="cuda")[offset:].view(m, kk)
+        losses._matmul_into(torch.empty(m, n, dtype=dtype, device="cuda"), a, torch.zeros(kk, n, dtype=dtype, device="cuda"))
+        return bool(calls)
+    assert try_(8, 64, 1 << 14) and try_(8, 68, 20008)
+    assert not try_(8, 64, 8192) and not try_(8, 66, 1 << 14) and not try_(8, 64, 20004)
+    assert not try_(8, 64, 1 << 14, torch.float32) and not try_(8, 64, 1 << 14, offset=4)
+    assert not try_(2056, 2048, 1 << 14)
