@@ -25,7 +25,8 @@
 // 640-byte record of the same masters and the m codes (two 16-byte and one 8-byte access).
 //
 // Segment descriptors travel in the kernel arguments when a call has at most
-// kInline segments (the per-parameter hook path: no copy at all), otherwise in
+// kInline segments (the per-parameter hook path: no copy at all) or, in a shorter
+// form, at most kTiny of interleaved state with the same coefficients; otherwise in
 // a device table filled by one asynchronous copy from a pinned staging slot.
 
 #include <hip/hip_runtime.h>
@@ -86,16 +87,49 @@ struct DevSeg {
 static_assert(sizeof(DevSeg) == 144, "DevSeg layout");
 constexpr uint32_t kVec = 1u, kSR = 2u, kPrev = 4u, kFastDiv = 8u, kVec4 = 16u;
 
+// A segment of a compact launch: interleaved state updated in place, coefficients shared with the rest.
+struct TinySeg {
+    void* p;
+    const void* g;
+    void* out;
+    uint32_t n;
+    uint32_t bits;         // flags, and n - n_main from bit kTailShift up
+    uint32_t idx0;
+    uint32_t seed_m;       // the other streams' seeds follow from it
+    int32_t tile_begin;
+    uint32_t pad;
+};
+static_assert(sizeof(TinySeg) == 48, "TinySeg layout");
+constexpr int kTailShift = 8;
+constexpr uint32_t kSaltV = 0xA511E9B3u, kSaltP = 0x6C8E9CF5u;   // kernels.c:164-165
+
+// Segments carried in the arguments of a compact launch: 78 descriptors of 48 bytes are what they hold.
+// A table costs the host an upload, two events and a wait, and the launch waits for the upload: 74 tensors
+// of a small decoder (6.8M parameters, FP32 records) took 84 us a step with a table, 47 so.
+constexpr int kTiny = 78;
+// More segments go as several such launches while the host is what takes the time: up to kTinySplit
+// launches, and up to kSplitElems elements (rounded up to tiles).  Repeated steps of BF16 pairs, one table
+// against launches of 78: 80 tensors of 3.6M elements 84 / 55 us, 150 of 20M 114 / 85, 290 of 38M 170 / 150,
+// 150 of 89M 301 / 299; 290 of 316M 1028 / 1036 (each launch's last wave).
+constexpr int kTinySplit = 4;
+constexpr int64_t kSplitElems = (int64_t)1 << 27;
+
 struct Launch {
-    const DevSeg* table;     // device table when nsegs > kInline
+    const DevSeg* table;     // device table when nsegs > kInline, or null: a compact launch
     const int64_t* starts;   // device: first tile of each segment (compact, for the search)
     int64_t tile;            // elements per tile (multiple of the kernel family's quantum)
     int64_t ntiles;          // tiles of the launch; the grid is ntiles rounded up to a multiple of 8
     int32_t nsegs;
     int32_t pad;
-    DevSeg inl[kInline];
+    union {
+        DevSeg inl[kInline];
+        struct {
+            Coef c;
+            TinySeg seg[kTiny];
+        } tiny;
+    };
 };
-static_assert(sizeof(Launch) <= 1024 + 64, "kernel argument block");
+static_assert(sizeof(Launch) <= 4096 - 256, "kernel argument block");
 
 constexpr int kXcds = 8;
 
@@ -119,6 +153,29 @@ __device__ __forceinline__ DevSeg load_desc(const ABH_CONST DevSeg* p)
     return u.s;
 }
 
+// A compact launch's segment as a descriptor (scalar loads and arithmetic).
+__device__ __forceinline__ DevSeg expand(const Launch& L, const ABH_CONST TinySeg* q)
+{
+    DevSeg s;
+    s.p = q->p;
+    s.p_lo = static_cast<uint8_t*>(s.p);
+    s.g = q->g;
+    s.out = q->out;
+    s.m = s.v = nullptr;
+    s.m_scale = s.v_scale = nullptr;
+    s.n = q->n;
+    s.n_main = s.n - (q->bits >> kTailShift);
+    s.tile_begin = q->tile_begin;
+    s.idx0 = q->idx0;
+    s.flags = q->bits & ((1u << kTailShift) - 1u);
+    const ABH_CONST Coef* c = (const ABH_CONST Coef*)&L.tiny.c;
+    s.c = Coef{c->b1, c->b2, c->omb1, c->omb2, c->decay, c->step, c->isbc2, c->eps};
+    s.seed_m = q->seed_m;
+    s.seed_v = hash32(s.seed_m ^ kSaltV);
+    s.seed_p = hash32(s.seed_m ^ kSaltP);
+    return s;
+}
+
 // The descriptor of the segment holding `tile`: binary search of the first-tile table, all
 // through scalar loads (uniform address, constant address space), result in scalar registers.
 __device__ __forceinline__ DevSeg find_segment(const Launch& L, int64_t tile)
@@ -131,6 +188,14 @@ __device__ __forceinline__ DevSeg find_segment(const Launch& L, int64_t tile)
             if (inl[mid].tile_begin <= tile) lo = mid; else hi = mid - 1;
         }
         return load_desc(inl + lo);
+    }
+    if (L.table == nullptr) {
+        const ABH_CONST TinySeg* tiny = (const ABH_CONST TinySeg*)&L.tiny.seg[0];
+        while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if (tiny[mid].tile_begin <= tile) lo = mid; else hi = mid - 1;
+        }
+        return expand(L, tiny + lo);
     }
     const ABH_CONST int64_t* starts = (const ABH_CONST int64_t*)L.starts;
     while (lo < hi) {

@@ -283,8 +283,8 @@ ADAMBRIDGE_API void adambridge_pool_set_spin(void* pool, int32_t spin);
  * are planned in full first (one per kernel variant, split where a variant has
  * more segments than a staging slot holds or more tiles than one dispatch
  * takes), so no size limit is met after something was enqueued.  A launch of
- * more than 7 segments stages its segment table through a reused pinned host
- * slot: on a stream under graph capture such a call returns ADAMBRIDGE_ECAPTURE
+ * more than 7 segments may stage its segment table through a reused pinned host
+ * slot: on a stream under graph capture every such call returns ADAMBRIDGE_ECAPTURE
  * before enqueueing anything. */
 ADAMBRIDGE_API int adambridge_multi_step(void* pool, adambridge_segment* const* segs, int32_t nsegs,
                                          int32_t threads);
@@ -318,8 +318,8 @@ ADAMBRIDGE_API const char* adambridge_backend(void);
  * results as adambridge_multi_step, enqueued on `stream` (a hipStream_t of the current device;
  * NULL: the null stream).  Instead of a pool's staging buffers it uses one static device array of
  * the library, 152 KiB per GPU, held until the process ends: launches of more than 7 segments of
- * one kernel variant find their segment table there, written by small kernels whose arguments
- * carry the descriptors (no copy from host memory).  Limit: 1024 segments per call (more:
+ * one kernel variant whose descriptors their arguments cannot carry find their segment table
+ * there, written by small kernels whose arguments do (no copy from host memory).  Limit: 1024 segments per call (more:
  * ADAMBRIDGE_ETOOMANY, with the reason in adambridge_last_error(), before anything is enqueued).
  * Every call on one GPU shares that GPU's array: calls that overlap on one GPU (other streams,
  * other threads, or replays of graphs holding such calls) race and must be ordered by the caller;
@@ -333,7 +333,8 @@ ADAMBRIDGE_API int adambridge_multi_step_noalloc(void* stream, adambridge_segmen
  * four values to rows[4k .. 4k + 3] while k < cap: the launch's number, its kernel variant, the
  * entry's first tile (negative where a segment continues from the previous launch) and the
  * launch's tile count.  A segment appears once, or once per launch its tiles are spread over when
- * they exceed one dispatch (2^32 - 1 work-items).  Returns the number of entries (which may
+ * they exceed one dispatch (2^32 - 1 work-items).  A launch of 79 to 312 short segments may be
+ * dispatched in up to four parts.  Returns the number of entries (which may
  * exceed cap), or a negative code. */
 ADAMBRIDGE_API int adambridge_plan_launches(adambridge_segment* const* segs, int32_t nsegs, int64_t* rows,
                                             int32_t cap);
