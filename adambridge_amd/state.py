@@ -419,6 +419,21 @@ class _Interleaved(ParamState):
         return master, total - master
 
 
+def _unit_scales(blocks: list[int], roles: tuple[str, ...], device) -> list[dict[str, torch.Tensor]]:
+    """FP8 block scales, all one, for states of ``blocks`` blocks: 256-byte-aligned parts of one allocation,
+    filled in one launch (two launches a state were 22 of 34 when a checkpoint of 11 tensors became FP8
+    state: 56 us of 760, and the gaps between them)."""
+    places, total = [], 0
+    for n in blocks:
+        mine = {}
+        for role in roles:
+            mine[role] = total
+            total += -(-n // 64) * 64
+        places.append(mine)
+    room = torch.ones(total, dtype=torch.float32, device=device)
+    return [{r: room[at: at + n] for r, at in mine.items()} for n, mine in zip(blocks, places)]
+
+
 class PairState(_Interleaved):
     """AdamW, FP32 master, BF16 moments: 16 bytes per pair of elements {p[2k], p[2k+1], m[2k] | m[2k+1] << 16,
     v[2k] | v[2k+1] << 16} (ADAMBRIDGE_DT_PACKED)."""
@@ -773,12 +788,13 @@ class AdamRecordState(_Interleaved):
     CODE = _hip.DT_PACKED8
     precision = "fp8"
 
-    def __init__(self, numel, device, double_buffer: bool = False, memory: list[torch.Tensor] | None = None):
+    def __init__(self, numel, device, double_buffer: bool = False, memory: list[torch.Tensor] | None = None,
+                 scales: dict[str, torch.Tensor] | None = None):
         self.blocks = F.fp8_blocks(int(numel))
         rec = memory[0].view(self.blocks, 768) if memory else \
             torch.zeros(self.blocks, 768, dtype=torch.uint8, device=device)
         super().__init__(numel, device, ("m", "v"), [rec])   # updated in place: never double-buffered
-        self.scales = {r: torch.ones(self.blocks, dtype=torch.float32, device=device) for r in ("m", "v")}
+        self.scales = scales or _unit_scales([self.blocks], ("m", "v"), device)[0]
 
     @staticmethod
     def buffer_bytes(numel: int) -> int:
@@ -842,12 +858,13 @@ class AdamF24RecordState(AdamRecordState):
     master_precision = "fp24"
     RECORD = 640
 
-    def __init__(self, numel, device, double_buffer: bool = False, memory: list[torch.Tensor] | None = None):
+    def __init__(self, numel, device, double_buffer: bool = False, memory: list[torch.Tensor] | None = None,
+                 scales: dict[str, torch.Tensor] | None = None):
         self.blocks = F.fp8_blocks(int(numel))
         rec = memory[0].view(self.blocks, self.RECORD) if memory else \
             torch.zeros(self.blocks, self.RECORD, dtype=torch.uint8, device=device)
         _Interleaved.__init__(self, numel, device, ("m", "v"), [rec])   # updated in place: never double-buffered
-        self.scales = {r: torch.ones(self.blocks, dtype=torch.float32, device=device) for r in ("m", "v")}
+        self.scales = scales or _unit_scales([self.blocks], ("m", "v"), device)[0]
 
     @staticmethod
     def buffer_bytes(numel: int) -> int:
@@ -908,12 +925,13 @@ class LionFP8RecordState(AdamRecordState):
     CODE = _hip.DT_PACKED8_LION
     RECORD = 640   # master_plane's record stride too
 
-    def __init__(self, numel, device, double_buffer: bool = False, memory: list[torch.Tensor] | None = None):
+    def __init__(self, numel, device, double_buffer: bool = False, memory: list[torch.Tensor] | None = None,
+                 scales: dict[str, torch.Tensor] | None = None):
         self.blocks = F.fp8_blocks(int(numel))
         rec = memory[0].view(self.blocks, self.RECORD) if memory else \
             torch.zeros(self.blocks, self.RECORD, dtype=torch.uint8, device=device)
         _Interleaved.__init__(self, numel, device, ("m",), [rec])   # updated in place: never double-buffered
-        self.scales = {"m": torch.ones(self.blocks, dtype=torch.float32, device=device)}
+        self.scales = scales or _unit_scales([self.blocks], ("m",), device)[0]
 
     @staticmethod
     def buffer_bytes(numel: int) -> int:
@@ -948,12 +966,13 @@ class LionFP8F24RecordState(AdamF24RecordState):
     CODE = _hip.DT_PACKED8_LION_F24
     RECORD = 512   # master_plane's record stride too
 
-    def __init__(self, numel, device, double_buffer: bool = False, memory: list[torch.Tensor] | None = None):
+    def __init__(self, numel, device, double_buffer: bool = False, memory: list[torch.Tensor] | None = None,
+                 scales: dict[str, torch.Tensor] | None = None):
         self.blocks = F.fp8_blocks(int(numel))
         rec = memory[0].view(self.blocks, self.RECORD) if memory else \
             torch.zeros(self.blocks, self.RECORD, dtype=torch.uint8, device=device)
         _Interleaved.__init__(self, numel, device, ("m",), [rec])   # updated in place: never double-buffered
-        self.scales = {"m": torch.ones(self.blocks, dtype=torch.float32, device=device)}
+        self.scales = scales or _unit_scales([self.blocks], ("m",), device)[0]
 
     @staticmethod
     def buffer_bytes(numel: int) -> int:
@@ -1098,9 +1117,10 @@ def new_states(layout: str, algorithm: str, precision: str, master_precision: st
     sizes = [t.numel() for t in masters]
     if memory is None:
         memory = arena_memory(layout, sizes, device, double_buffer, place)
+    scales = _unit_scales([F.fp8_blocks(n) for n in sizes], roles, device) if cls.precision == "fp8" else None
     states = []
-    for n, mem, values in zip(sizes, memory, masters):
-        state = cls(n, device, double_buffer, memory=mem)
+    for i, (n, mem, values) in enumerate(zip(sizes, memory, masters)):
+        state = cls(n, device, double_buffer, memory=mem, **({"scales": scales[i]} if scales else {}))
         if fill:
             state.load(master=values.detach().reshape(-1))   # bf16 or fp32, read as it is by the kernel
         states.append(state)
