@@ -100,6 +100,13 @@ struct TinySeg {
     uint32_t pad;
 };
 static_assert(sizeof(TinySeg) == 48, "TinySeg layout");
+// The same with the block scales of an FP8 record.
+struct TinySeg8 {
+    TinySeg t;
+    float* m_scale;
+    float* v_scale;
+};
+static_assert(sizeof(TinySeg8) == 64, "TinySeg8 layout");
 constexpr int kTailShift = 8;
 constexpr uint32_t kSaltV = 0xA511E9B3u, kSaltP = 0x6C8E9CF5u;   // kernels.c:164-165
 
@@ -107,12 +114,14 @@ constexpr uint32_t kSaltV = 0xA511E9B3u, kSaltP = 0x6C8E9CF5u;   // kernels.c:16
 // A table costs the host an upload, two events and a wait, and the launch waits for the upload: 74 tensors
 // of a small decoder (6.8M parameters, FP32 records) took 84 us a step with a table, 47 so.
 constexpr int kTiny = 78;
+constexpr int kTiny8 = 58;   // FP8 records: 64 bytes each
 // More segments go as several such launches while the host is what takes the time: up to kTinySplit
 // launches, and up to kSplitElems elements (rounded up to tiles).  Repeated steps of BF16 pairs, one table
 // against launches of 78: 80 tensors of 3.6M elements 84 / 55 us, 150 of 20M 114 / 85, 290 of 38M 170 / 150,
-// 150 of 89M 301 / 299; 290 of 316M 1028 / 1036 (each launch's last wave).
+// 150 of 89M 301 / 299; 290 of 316M 1028 / 1036 (each launch's last wave).  FP8 records: 40 tensors of 1.8M
+// 71 / 37, 74 of 9.8M 86 / 53, 150 of 20M 121 / 89; 150 of 89M 257 / 260.
 constexpr int kTinySplit = 4;
-constexpr int64_t kSplitElems = (int64_t)1 << 27;
+constexpr int64_t kSplitElems = (int64_t)1 << 26;
 
 struct Launch {
     const DevSeg* table;     // device table when nsegs > kInline, or null: a compact launch
@@ -127,6 +136,10 @@ struct Launch {
             Coef c;
             TinySeg seg[kTiny];
         } tiny;
+        struct {
+            Coef c;
+            TinySeg8 seg[kTiny8];
+        } tiny8;
     };
 };
 static_assert(sizeof(Launch) <= 4096 - 256, "kernel argument block");
@@ -158,7 +171,7 @@ __device__ __forceinline__ DevSeg expand(const Launch& L, const ABH_CONST TinySe
 {
     DevSeg s;
     s.p = q->p;
-    s.p_lo = static_cast<uint8_t*>(s.p);
+    s.p_lo = static_cast<uint8_t*>(s.p);   // updated in place
     s.g = q->g;
     s.out = q->out;
     s.m = s.v = nullptr;
@@ -178,6 +191,7 @@ __device__ __forceinline__ DevSeg expand(const Launch& L, const ABH_CONST TinySe
 
 // The descriptor of the segment holding `tile`: binary search of the first-tile table, all
 // through scalar loads (uniform address, constant address space), result in scalar registers.
+template <bool FP8 = false>
 __device__ __forceinline__ DevSeg find_segment(const Launch& L, int64_t tile)
 {
     int lo = 0, hi = L.nsegs - 1;
@@ -189,7 +203,19 @@ __device__ __forceinline__ DevSeg find_segment(const Launch& L, int64_t tile)
         }
         return load_desc(inl + lo);
     }
-    if (L.table == nullptr) {
+    if (FP8 && L.table == nullptr) {
+        const ABH_CONST TinySeg8* tiny = (const ABH_CONST TinySeg8*)&L.tiny8.seg[0];
+        while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if (tiny[mid].t.tile_begin <= tile) lo = mid; else hi = mid - 1;
+        }
+        DevSeg s = expand(L, &tiny[lo].t);   // the coefficients lie where L.tiny's do
+        s.p_lo = nullptr;
+        s.m_scale = tiny[lo].m_scale;
+        s.v_scale = tiny[lo].v_scale;
+        return s;
+    }
+    if (!FP8 && L.table == nullptr) {
         const ABH_CONST TinySeg* tiny = (const ABH_CONST TinySeg*)&L.tiny.seg[0];
         while (lo < hi) {
             const int mid = (lo + hi + 1) >> 1;
@@ -1137,7 +1163,7 @@ __global__ __launch_bounds__(kThreads) void k_update_fp8(Launch L)
 {
     const int64_t tile = block_tile(L);
     if (tile >= L.ntiles) return;
-    const DevSeg s = find_segment(L, tile);
+    const DevSeg s = find_segment<true>(L, tile);
     // the out-from-previous-master form is its own instantiation: a runtime test inside the block
     // code cost this VALU-heavy kernel 6% (measured on the 7B FP8 step)
     if (s.flags & kPrev) {

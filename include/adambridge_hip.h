@@ -333,7 +333,7 @@ ADAMBRIDGE_API int adambridge_multi_step_noalloc(void* stream, adambridge_segmen
  * four values to rows[4k .. 4k + 3] while k < cap: the launch's number, its kernel variant, the
  * entry's first tile (negative where a segment continues from the previous launch) and the
  * launch's tile count.  A segment appears once, or once per launch its tiles are spread over when
- * they exceed one dispatch (2^32 - 1 work-items).  A launch of 79 to 312 short segments may be
+ * they exceed one dispatch (2^32 - 1 work-items).  A launch of 59 to 312 small segments may be
  * dispatched in up to four parts.  Returns the number of entries (which may
  * exceed cap), or a negative code. */
 ADAMBRIDGE_API int adambridge_plan_launches(adambridge_segment* const* segs, int32_t nsegs, int64_t* rows,

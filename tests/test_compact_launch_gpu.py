@@ -9,7 +9,7 @@ import torch
 
 from adambridge_amd import _hip
 from hip_cases import (run_hip_f24_records, run_hip_f32_records, run_hip_lion_f32_records, run_hip_lion_records,
-                       run_hip_packed)
+                       run_hip_packed, run_hip_records)
 from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -19,19 +19,22 @@ LAYOUTS = {"pairs": (run_hip_packed, dict(mv_dtype=O.DT_BF16)),
            "f32": (run_hip_f32_records, dict(mv_dtype=O.DT_F32)),
            "lion-f32": (run_hip_lion_f32_records, dict(algorithm=O.LION, mv_dtype=O.DT_F32)),
            "f24": (run_hip_f24_records, dict(mv_dtype=O.DT_BF16, p_dtype=O.DT_F24)),
+           "fp8": (run_hip_records, dict(mv_dtype=O.DT_FP8)),
+           "fp8-f24": (run_hip_records, dict(mv_dtype=O.DT_FP8, p_dtype=O.DT_F24)),
+           "lion-fp8": (run_hip_records, dict(algorithm=O.LION, mv_dtype=O.DT_FP8)),
            "lion-f24-f32": (run_hip_f24_records, dict(algorithm=O.LION, mv_dtype=O.DT_F32, p_dtype=O.DT_F24))}
 
 
-# 7 fit as full descriptors, 8 to 78 in the short form, up to 312 in several such launches, 313 need a
-# table, and so does one segment with other coefficients among 20; several tiles and scalar tails
-@pytest.mark.parametrize("count,odd", [(7, None), (8, None), (78, None), (79, None), (157, None), (312, None),
+# 7 fit as full descriptors, 8 to 78 (FP8: 58) in the short form, up to 312 (232) in several such launches,
+# more need a table, and so does one segment with other coefficients among 20; several tiles and scalar tails
+@pytest.mark.parametrize("count,odd", [(7, None), (8, None), (78, None), (79, None), (157, None), (312, None), (58, None), (59, None), (232, None),
                                        (313, None), (20, 0), (20, 19)])
 @pytest.mark.parametrize("layout", list(LAYOUTS))
 def test_segment_counts_match_oracle(layout, count, odd):
     run, kw = LAYOUTS[layout]
     rng = np.random.default_rng(count)
     sizes = [1, 127, 128, 129, 40001, 255, 5000] + [int(n) for n in rng.integers(1, 6000, count)]
-    cases = [O.make_case(rng, sizes[k], index=7 * k, offset=int(rng.integers(0, 2**32)), step=4 if k == odd else 3,
+    cases = [O.make_case(rng, sizes[k], index=7 * k, offset=128 * int(rng.integers(0, 2**25)), step=4 if k == odd else 3,
                          stochastic=k % 3 != 0, **kw) for k in range(count)]
     for width in (16, 0):
         for flags in (0, 1):   # 1: out receives the weight from before the update
