@@ -94,8 +94,8 @@ def _matmul_into(out: torch.Tensor, a: torch.Tensor, b: torch.Tensor) -> None:
     """``out`` = ``a @ b``: by the library's split product (csrc/abh_gemm.hip) where the inner dimension is long
     and the result small -- there the BLAS library leaves most of the chip idle -- else by torch."""
     (m, k), n = a.shape, b.shape[1]
-    if (a.dtype == torch.bfloat16 and 1 << 14 <= k <= 1 << 22 and m * n <= 1 << 22 and n % 4 == 0 and k % 8 == 0
-            and a.data_ptr() % 16 == 0 and b.data_ptr() % 8 == 0 and out.data_ptr() % 8 == 0):
+    if (a.dtype == b.dtype == out.dtype == torch.bfloat16 and 1 << 14 <= k <= 1 << 22 and m * n <= 1 << 22
+            and n % 4 == 0 and k % 8 == 0 and a.data_ptr() % 16 == 0 and b.data_ptr() % 8 == 0 and out.data_ptr() % 8 == 0):
         _hip.load().matmul(a, b, out)
     else:
         torch.mm(a, b, out=out)
@@ -124,25 +124,26 @@ class _HeadLoss(torch.autograd.Function):
     def backward(ctx, gout):
         h, weight, targets, *kept = ctx.saved_tensors
         wanted = ctx.needs_input_grad[:2]
-        if torch.is_grad_enabled():   # create_graph: gradients that are differentiated in turn
-            total = sum(_torch_loss_sum(torch.mm(a, weight.t()), t, ctx.ignore_index)
-                        for a, t in zip(torch.split(h, ctx.chunk), torch.split(targets, ctx.chunk)))
-            inputs = [x for x, want in zip((h, weight), wanted) if want]
-            grads = iter(torch.autograd.grad(total, inputs, gout, create_graph=True))
-            return (*(next(grads) if want else None for want in wanted), None, None, None)
-        k = _hip.load()
-        dh = torch.empty_like(h) if wanted[0] else None
-        dw = None
-        parts = zip(torch.split(h, ctx.chunk), torch.split(targets, ctx.chunk), kept,
-                    torch.split(h if dh is None else dh, ctx.chunk))
-        for h_part, t_part, stats, dh_part in parts:
-            logits = torch.mm(h_part, weight.t())
-            grad = k.cross_entropy_backward(logits, t_part, ctx.ignore_index, stats, gout, out=logits)
-            if wanted[0]:
-                _matmul_into(dh_part, grad, weight)
-            if wanted[1]:
-                dw = torch.mm(grad.t(), h_part) if dw is None else dw.addmm_(grad.t(), h_part)
-            del logits, grad
+        with torch.autocast(h.device.type, enabled=False):   # as the forward ran (_head_applies)
+            if torch.is_grad_enabled():   # create_graph: gradients that are differentiated in turn
+                total = sum(_torch_loss_sum(torch.mm(a, weight.t()), t, ctx.ignore_index)
+                            for a, t in zip(torch.split(h, ctx.chunk), torch.split(targets, ctx.chunk)))
+                inputs = [x for x, want in zip((h, weight), wanted) if want]
+                grads = iter(torch.autograd.grad(total, inputs, gout, create_graph=True))
+                return (*(next(grads) if want else None for want in wanted), None, None, None)
+            k = _hip.load()
+            dh = torch.empty_like(h) if wanted[0] else None
+            dw = None
+            parts = zip(torch.split(h, ctx.chunk), torch.split(targets, ctx.chunk), kept,
+                        torch.split(h if dh is None else dh, ctx.chunk))
+            for h_part, t_part, stats, dh_part in parts:
+                logits = torch.mm(h_part, weight.t())
+                grad = k.cross_entropy_backward(logits, t_part, ctx.ignore_index, stats, gout, out=logits)
+                if wanted[0]:
+                    _matmul_into(dh_part, grad, weight)
+                if wanted[1]:
+                    dw = torch.mm(grad.t(), h_part) if dw is None else dw.addmm_(grad.t(), h_part)
+                del logits, grad
         return dh, dw, None, None, None
 
 

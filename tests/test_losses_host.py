@@ -1,0 +1,101 @@
+"""causal_lm_loss's choice between the library's kernels and torch operations, and its backward passes'
+surroundings, on the CPU: the kernels are stood in for by torch operations that refuse any operand the
+real ones could not take."""
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+import adambridge_amd as ab
+from adambridge_amd import _hip, losses
+
+IGNORE = -100
+
+
+class Kernels:
+    """HipKernels' loss calls in torch operations on host tensors; ``calls`` names each one made."""
+
+    def __init__(self):
+        self.calls = []
+
+    def cross_entropy(self, logits, target, ignore_index):
+        self.calls.append("cross_entropy")
+        assert type(logits) is torch.Tensor and logits.dtype in (torch.float32, torch.bfloat16)
+        logits.data_ptr()
+        x = logits.detach().float()
+        m = x.amax(1)
+        s = (x - m[:, None]).exp().sum(1)
+        at = target.clamp(0, x.shape[1] - 1)[:, None]
+        terms = torch.where(target == ignore_index, 0.0, s.log() - (x.gather(1, at)[:, 0] - m))
+        return terms.sum(), torch.stack((m, 1.0 / s), 1)
+
+    def cross_entropy_backward(self, logits, target, ignore_index, stats, gout, out=None):
+        self.calls.append("cross_entropy_backward")
+        assert gout.dtype == torch.float32 and gout.numel() == 1
+        logits.data_ptr(), gout.data_ptr()
+        g = torch.where(target == ignore_index, 0.0, gout)[:, None]
+        p = (logits.detach().float() - stats[:, :1]).exp() * stats[:, 1:] * g
+        p.scatter_add_(1, target.clamp(0, p.shape[1] - 1)[:, None], -g)
+        out = torch.empty_like(logits) if out is None else out
+        assert out.dtype == logits.dtype and out.shape == logits.shape
+        return out.copy_(p)
+
+    def matmul(self, a, b, out):
+        self.calls.append("matmul")
+        assert a.dtype == b.dtype == out.dtype == torch.bfloat16
+        out.copy_(a.float() @ b.float())
+
+
+@pytest.fixture
+def kernels(monkeypatch):
+    """The stand-ins, taken for host tensors as the real ones are for tensors on a GPU."""
+    def ordinary(values, target):
+        return (type(target) is torch.Tensor and values.dtype in (torch.bfloat16, torch.float32)
+                and target.dtype == torch.int64 and values.dim() == 2 and target.dim() == 1
+                and target.numel() == values.shape[0] and values.is_contiguous() and target.is_contiguous()
+                and values.numel() > 0)
+
+    k = Kernels()
+    monkeypatch.setattr(_hip, "load", lambda: k)
+    monkeypatch.setattr(losses, "_ordinary", ordinary)
+    return k
+
+
+def _problem(dtype=torch.float32, vocab=61, bias=False, seed=1):
+    gen = torch.Generator().manual_seed(seed)
+    hidden = torch.randn(2, 12, 8, generator=gen).to(dtype).requires_grad_()
+    head = torch.nn.Linear(8, vocab, bias=bias, dtype=dtype)
+    with torch.no_grad():
+        for p in head.parameters():
+            p.copy_(torch.randn(p.shape, generator=gen) * 0.4)
+    labels = torch.randint(0, vocab, (2, 12), generator=gen)
+    labels[:, :3] = IGNORE
+    return hidden, head, labels
+
+
+def _loss(hidden, head, labels, chunk=10):
+    return ab.causal_lm_loss(hidden, head, labels, chunk_tokens=chunk)
+
+
+def _whole(hidden, head, labels):
+    """The same loss in plain torch operations."""
+    return F.cross_entropy(head(hidden[:, :-1]).flatten(0, 1).float(), labels[:, 1:].flatten(), ignore_index=IGNORE)
+
+
+def _close(got, want, rel=1e-5):
+    return all((a - b).norm() <= rel * b.norm() for a, b in zip(got, want, strict=True))
+
+
+@pytest.mark.parametrize("chunk", [10, 100])
+@pytest.mark.parametrize("vocab", [61, 1 << 14])   # the hidden gradient by torch's product, by the split one's rule
+@pytest.mark.parametrize("frozen", [False, True])
+def test_backward_under_autocast_keeps_the_forwards_types(kernels, vocab, chunk, frozen):
+    hidden, head, labels = _problem(vocab=vocab)
+    head.weight.requires_grad_(not frozen)
+    inputs = [hidden] if frozen else [hidden, head.weight]
+    want = torch.autograd.grad(_whole(hidden, head, labels), inputs)
+    loss = _loss(hidden, head, labels, chunk)
+    with torch.autocast("cpu", dtype=torch.bfloat16):
+        got = torch.autograd.grad(loss, inputs)
+    assert "cross_entropy_backward" in kernels.calls
+    assert all(g.dtype == torch.float32 for g in got) and _close(got, want)
