@@ -103,26 +103,28 @@ def _matmul_into(out: torch.Tensor, a: torch.Tensor, b: torch.Tensor) -> None:
 
 class _HeadLoss(torch.autograd.Function):
     """Summed cross-entropy of ``h @ weight.T``, ``chunk`` rows at a time.  The backward pass computes each
-    slice's logits again, as the checkpointed slices do, but neither their statistics (two floats per
-    row, kept) nor a gradient beside them (it takes the logits' place), and the weight's gradient is
-    added up inside the products (rounded once per slice, where the slices' gradients were each
-    rounded, then added and rounded)."""
+    slice's logits again, as the checkpointed slices do, but no gradient beside them (it takes the
+    logits' place), and the weight's gradient is added up inside the products (rounded once per slice,
+    where the slices' gradients were each rounded, then added and rounded).
+
+    The weight may have been written meanwhile (an optimizer step between two losses' backward passes;
+    the update kernels write it without a version count): as in the checkpointed slices, the
+    gradient is then that at the weight as it is, so the rows' statistics are taken from the logits
+    computed again, and the weight is held by reference, not as a saved tensor."""
 
     @staticmethod
     def forward(ctx, h, weight, targets, ignore_index, chunk):
         k = _hip.load()
-        total, kept = h.new_zeros((), dtype=torch.float32), []
+        total = h.new_zeros((), dtype=torch.float32)
         for h_part, t_part in zip(torch.split(h, chunk), torch.split(targets, chunk)):
-            loss, stats = k.cross_entropy(torch.mm(h_part, weight.t()), t_part, ignore_index)
-            total += loss
-            kept.append(stats)
-        ctx.save_for_backward(h, weight, targets, *kept)
-        ctx.ignore_index, ctx.chunk = ignore_index, chunk
+            total += k.cross_entropy(torch.mm(h_part, weight.t()), t_part, ignore_index)[0]
+        ctx.save_for_backward(h, targets)
+        ctx.weight, ctx.ignore_index, ctx.chunk = weight, ignore_index, chunk
         return total
 
     @staticmethod
     def backward(ctx, gout):
-        h, weight, targets, *kept = ctx.saved_tensors
+        (h, targets), weight = ctx.saved_tensors, ctx.weight
         wanted = ctx.needs_input_grad[:2]
         with torch.autocast(h.device.type, enabled=False):   # as the forward ran (_head_applies)
             if torch.is_grad_enabled():   # create_graph: gradients that are differentiated in turn
@@ -134,10 +136,11 @@ class _HeadLoss(torch.autograd.Function):
             k = _hip.load()
             dh = torch.empty_like(h) if wanted[0] else None
             dw = None
-            parts = zip(torch.split(h, ctx.chunk), torch.split(targets, ctx.chunk), kept,
+            parts = zip(torch.split(h, ctx.chunk), torch.split(targets, ctx.chunk),
                         torch.split(h if dh is None else dh, ctx.chunk))
-            for h_part, t_part, stats, dh_part in parts:
+            for h_part, t_part, dh_part in parts:
                 logits = torch.mm(h_part, weight.t())
+                stats = k.cross_entropy(logits, t_part, ctx.ignore_index)[1]
                 grad = k.cross_entropy_backward(logits, t_part, ctx.ignore_index, stats, gout, out=logits)
                 if wanted[0]:
                     _matmul_into(dh_part, grad, weight)

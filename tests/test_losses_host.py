@@ -99,3 +99,23 @@ def test_backward_under_autocast_keeps_the_forwards_types(kernels, vocab, chunk,
         got = torch.autograd.grad(loss, inputs)
     assert "cross_entropy_backward" in kernels.calls
     assert all(g.dtype == torch.float32 for g in got) and _close(got, want)
+
+
+@pytest.mark.parametrize("counted", [True, False])   # written through torch, or as the update kernels write: no version
+def test_a_weight_written_between_the_passes_is_read_as_it_is(kernels, counted):
+    hidden, head, labels = _problem()
+    loss = _loss(hidden, head, labels)
+    new = head.weight.detach() * 40.0   # logits far above the first pass's row maxima
+    with torch.no_grad():
+        head.weight.copy_(new) if counted else head.weight.data.copy_(new)
+    got = torch.autograd.grad(loss, [hidden, head.weight])
+    assert "cross_entropy_backward" in kernels.calls
+    assert _close(got, torch.autograd.grad(_whole(hidden, head, labels), [hidden, head.weight]))
+
+
+def test_a_second_backward_needs_the_graph_kept(kernels):
+    hidden, head, labels = _problem()
+    loss = _loss(hidden, head, labels)
+    loss.backward()
+    with pytest.raises(RuntimeError, match="backward through the graph a second time"):
+        loss.backward()
