@@ -175,8 +175,9 @@ def causal_lm_loss(hidden_states: torch.Tensor, lm_head: Callable[[torch.Tensor]
     no target); the mean runs over positions whose target is not ``ignore_index`` -- the Hugging
     Face causal-LM loss.  ``hidden_states``: ``[batch, seq, hidden]``; ``lm_head``: a module or
     function mapping ``[n, hidden]`` to ``[n, vocab]``; ``labels``: ``[batch, seq]`` token ids.
-    With gradients enabled, each slice runs under non-reentrant ``torch.utils.checkpoint``, or (a
-    plain ``torch.nn.Linear`` head on the GPU) in one function of the same memory (:class:`_HeadLoss`).
+    With a gradient to the hidden states, each slice runs under non-reentrant ``torch.utils.checkpoint``,
+    or (a plain ``torch.nn.Linear`` head on the GPU) in one function of the same memory
+    (:class:`_HeadLoss`); with one to the head alone, the slices' logits are kept.
     """
     if hidden_states.dim() != 3:
         raise ValueError(f"hidden_states must be [batch, seq, hidden], got shape {tuple(hidden_states.shape)}")
@@ -191,9 +192,9 @@ def causal_lm_loss(hidden_states: torch.Tensor, lm_head: Callable[[torch.Tensor]
     targets[:, :-1] = labels[:, 1:]
     targets = targets.reshape(-1).to(h.device)
     n_scored = (targets != ignore_index).sum()
-    if torch.is_grad_enabled() and _head_applies(lm_head, h, targets) and (h.requires_grad or lm_head.weight.requires_grad):
-        return _HeadLoss.apply(h, lm_head.weight, targets, ignore_index, chunk_tokens) / n_scored.clamp(min=1)
     recompute = torch.is_grad_enabled() and h.requires_grad
+    if recompute and _head_applies(lm_head, h, targets):
+        return _HeadLoss.apply(h, lm_head.weight, targets, ignore_index, chunk_tokens) / n_scored.clamp(min=1)
     total = h.new_zeros((), dtype=torch.float32)
     for h_part, t_part in zip(torch.split(h, chunk_tokens), torch.split(targets, chunk_tokens)):
         if recompute:

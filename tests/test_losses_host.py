@@ -119,3 +119,14 @@ def test_a_second_backward_needs_the_graph_kept(kernels):
     loss.backward()
     with pytest.raises(RuntimeError, match="backward through the graph a second time"):
         loss.backward()
+
+
+def test_a_frozen_hidden_state_keeps_the_weights_gradient_of_the_forward_pass(kernels):
+    """Without a gradient to the hidden states nothing is computed again: the slices' logits are kept."""
+    hidden, head, labels = _problem()
+    hidden.requires_grad_(False)
+    want = torch.autograd.grad(_whole(hidden, head, labels), head.weight)
+    loss = _loss(hidden, head, labels)
+    head.weight.data.mul_(3.0)
+    assert _close(torch.autograd.grad(loss, head.weight), want)
+    assert "cross_entropy_backward" in kernels.calls
