@@ -47,9 +47,9 @@ def _ordinary(values: torch.Tensor, target: torch.Tensor) -> bool:
             and 0 < values.shape[0] <= _MAX_ROWS and values.shape[1] > 0)
 
 
-def _kernels_apply(logits: torch.Tensor, target: torch.Tensor) -> bool:
-    """Whether the library's cross-entropy takes this slice."""
-    return (not _observed() and type(logits) is torch.Tensor and _ordinary(logits, target)
+def _kernels_apply(logits: torch.Tensor, target: torch.Tensor, observed: bool | None = None) -> bool:
+    """Whether the library's cross-entropy takes this slice (``observed``: :func:`_observed`, if asked before)."""
+    return (not (_observed() if observed is None else observed) and type(logits) is torch.Tensor and _ordinary(logits, target)
             and logits.data_ptr() % 16 == 0)   # so that the gradient, a new tensor, shares its alignment
 
 
@@ -156,10 +156,12 @@ def _torch_loss_sum(logits: torch.Tensor, target: torch.Tensor, ignore_index: in
 
 
 def _slice_loss_sum(h: torch.Tensor, target: torch.Tensor, project: Callable[[torch.Tensor], torch.Tensor],
-                    ignore_index: int) -> torch.Tensor:
-    """Summed cross-entropy of one slice."""
+                    ignore_index: int, observed: bool | None = None) -> torch.Tensor:
+    """Summed cross-entropy of one slice.  A checkpointed slice is computed again in the backward pass, where
+    other modes may be active (the default device's is not, for one) but the same tensors must be
+    saved: its caller passes what it found ``observed``."""
     logits = project(h)
-    if not _kernels_apply(logits, target):
+    if not _kernels_apply(logits, target, observed):
         return _torch_loss_sum(logits, target, ignore_index)
     if torch.is_grad_enabled() and logits.requires_grad:
         return _SliceLoss.apply(logits, target, ignore_index)
@@ -195,10 +197,12 @@ def causal_lm_loss(hidden_states: torch.Tensor, lm_head: Callable[[torch.Tensor]
     recompute = torch.is_grad_enabled() and h.requires_grad
     if recompute and _head_applies(lm_head, h, targets):
         return _HeadLoss.apply(h, lm_head.weight, targets, ignore_index, chunk_tokens) / n_scored.clamp(min=1)
+    observed = _observed()
     total = h.new_zeros((), dtype=torch.float32)
     for h_part, t_part in zip(torch.split(h, chunk_tokens), torch.split(targets, chunk_tokens)):
         if recompute:
-            total = total + checkpoint(_slice_loss_sum, h_part, t_part, lm_head, ignore_index, use_reentrant=False)
+            total = total + checkpoint(_slice_loss_sum, h_part, t_part, lm_head, ignore_index, observed,
+                                       use_reentrant=False)
         else:
-            total = total + _slice_loss_sum(h_part, t_part, lm_head, ignore_index)
+            total = total + _slice_loss_sum(h_part, t_part, lm_head, ignore_index, observed)
     return total / n_scored.clamp(min=1)

@@ -130,3 +130,46 @@ def test_a_frozen_hidden_state_keeps_the_weights_gradient_of_the_forward_pass(ke
     head.weight.data.mul_(3.0)
     assert _close(torch.autograd.grad(loss, head.weight), want)
     assert "cross_entropy_backward" in kernels.calls
+
+
+class _Watch(torch.overrides.TorchFunctionMode):
+    def __torch_function__(self, func, types, args=(), kwargs=None):
+        return func(*args, **(kwargs or {}))
+
+
+def _modes():
+    from torch.utils.flop_counter import FlopCounterMode
+    return {"function": _Watch, "device": lambda: torch.device("cpu"), "flops": lambda: FlopCounterMode(display=False)}
+
+
+@pytest.mark.parametrize("head_kind", ["bias", "lambda", "linear"])
+@pytest.mark.parametrize("where", ["forward", "backward", "both"])
+@pytest.mark.parametrize("mode", ["function", "device", "flops"])
+def test_a_mode_around_either_pass(kernels, mode, where, head_kind):
+    """The choice between kernels and torch operations is the call's: what a checkpointed slice computes
+    again is what it computed first, whatever is active then."""
+    hidden, head, labels = _problem(bias=head_kind == "bias")
+    project = (lambda x: head(x)) if head_kind == "lambda" else head
+    inputs = [hidden, *head.parameters()]
+    want = torch.autograd.grad(_whole(hidden, head, labels), inputs)
+    from contextlib import nullcontext
+    make = _modes()[mode]
+    with make() if where != "backward" else nullcontext():
+        loss = ab.causal_lm_loss(hidden, project, labels, chunk_tokens=10)
+        if where == "both":
+            loss.backward()
+    with make() if where == "backward" else nullcontext():
+        if where != "both":
+            loss.backward()
+    assert _close([p.grad for p in inputs], want)
+
+
+def test_a_default_device_around_the_whole_step(kernels):
+    hidden, head, labels = _problem(bias=True)
+    want = torch.autograd.grad(_whole(hidden, head, labels), [hidden, *head.parameters()])
+    torch.set_default_device("cpu")
+    try:
+        _loss(hidden, head, labels).backward()
+    finally:
+        torch.set_default_device(None)
+    assert _close([hidden.grad, *(p.grad for p in head.parameters())], want)
