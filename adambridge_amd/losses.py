@@ -19,6 +19,7 @@ from typing import Callable
 import torch
 import torch.autograd.forward_ad as forward_ad
 import torch.nn.functional as F
+from torch.utils._device import DeviceContext
 from torch.utils.checkpoint import checkpoint
 
 from . import _hip
@@ -31,10 +32,12 @@ _MAX_ROWS = 1 << 23   # adambridge_cross_entropy's
 
 def _observed() -> bool:
     """Whether something needs the torch operations themselves: a trace or compilation, a function
-    transform (vmap, functorch grad), forward-mode derivatives, a mode that observes operations."""
+    transform (vmap, functorch grad), forward-mode derivatives, a mode that observes operations (a
+    default device does not: it is where factory calls that name no device put their tensors)."""
     return bool(torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._are_functorch_transforms_active()
                 or forward_ad._current_level >= 0 or torch._C._len_torch_dispatch_stack()
-                or torch._C._len_torch_function_stack())
+                or any(not isinstance(torch._C._get_function_stack_at(i), DeviceContext)
+                       for i in range(torch._C._len_torch_function_stack())))
 
 
 def _ordinary(values: torch.Tensor, target: torch.Tensor) -> bool:
@@ -158,7 +161,7 @@ def _torch_loss_sum(logits: torch.Tensor, target: torch.Tensor, ignore_index: in
 def _slice_loss_sum(h: torch.Tensor, target: torch.Tensor, project: Callable[[torch.Tensor], torch.Tensor],
                     ignore_index: int, observed: bool | None = None) -> torch.Tensor:
     """Summed cross-entropy of one slice.  A checkpointed slice is computed again in the backward pass, where
-    other modes may be active (the default device's is not, for one) but the same tensors must be
+    other modes may be active but the same tensors must be
     saved: its caller passes what it found ``observed``."""
     logits = project(h)
     if not _kernels_apply(logits, target, observed):

@@ -173,3 +173,23 @@ def test_a_default_device_around_the_whole_step(kernels):
     finally:
         torch.set_default_device(None)
     assert _close([hidden.grad, *(p.grad for p in head.parameters())], want)
+
+
+@pytest.mark.parametrize("bias", [False, True])
+def test_a_default_device_does_not_keep_the_kernels_away(kernels, bias):
+    """A default device changes where factories put new tensors, and is there for a whole program."""
+    hidden, head, labels = _problem(bias=bias)
+    torch.set_default_device("cpu")
+    try:
+        _loss(hidden, head, labels).backward()
+        assert kernels.calls.count("cross_entropy_backward") == 3
+        kernels.calls.clear()
+        with torch.no_grad():
+            _loss(hidden, head, labels)
+        assert kernels.calls == ["cross_entropy"] * 3
+        kernels.calls.clear()
+        with _Watch():
+            _loss(hidden, head, labels).backward()
+        assert not kernels.calls
+    finally:
+        torch.set_default_device(None)
