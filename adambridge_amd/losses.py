@@ -73,23 +73,47 @@ def _head_applies(head, h: torch.Tensor, targets: torch.Tensor) -> bool:
             and w.is_contiguous() and not w.is_neg() and w.shape[1] == h.shape[1] and w.shape[0] > 0)
 
 
+def _plain_backward(gout: torch.Tensor) -> bool:
+    """Whether this backward pass may run the kernels: not one that is differentiated in turn (create_graph)
+    or observed, nor one whose incoming gradient is a batch (is_grads_batched) or otherwise holds no memory."""
+    return (not torch.is_grad_enabled() and not _observed() and type(gout) is torch.Tensor
+            and torch._C._has_storage(gout) and not gout._is_zerotensor())
+
+
+def _logits_gradient(logits: torch.Tensor, target: torch.Tensor, ignore_index: int, gout: torch.Tensor) -> torch.Tensor:
+    """What ``cross_entropy_backward`` computes, in torch operations: differentiable, and for a ``gout`` that is
+    a batch (vmap)."""
+    p = logits.float().softmax(1)
+    seed = torch.where(target == ignore_index, 0.0, gout)[:, None]   # an ignored row: 0 times what it holds
+    at = target.clamp(0, logits.shape[1] - 1)[:, None]
+    return (p.scatter_add(1, at, p.new_full((), -1.0).expand_as(at)) * seed).to(logits.dtype)
+
+
 class _SliceLoss(torch.autograd.Function):
-    """Summed cross-entropy by the library's kernels.  What is kept for the backward pass is the logits
-    themselves and two floats per row."""
+    """Summed cross-entropy by the library's kernels, and the two floats per row that are kept for the
+    backward pass beside the logits themselves.  (Forward and context apart: a checkpointed slice may be
+    computed again while a batched backward pass runs under vmap, on tensors that are not batched.)"""
 
     @staticmethod
-    def forward(ctx, logits, target, ignore_index):
-        loss, stats = _hip.load().cross_entropy(logits, target, ignore_index)
-        ctx.save_for_backward(logits, target, stats)
-        ctx.ignore_index = ignore_index
-        return loss
+    def forward(logits, target, ignore_index):
+        return _hip.load().cross_entropy(logits, target, ignore_index)
 
     @staticmethod
-    def backward(ctx, gout):
+    def setup_context(ctx, inputs, output):
+        logits, target, ctx.ignore_index = inputs
+        ctx.save_for_backward(logits, target, output[1])
+        ctx.mark_non_differentiable(output[1])
+        ctx.set_materialize_grads(False)
+
+    @staticmethod
+    def vmap(info, in_dims, logits, target, ignore_index):
+        raise NotImplementedError("batched logits take the torch operations (_kernels_apply)")
+
+    @staticmethod
+    def backward(ctx, gout, _):
         logits, target, stats = ctx.saved_tensors
-        if torch.is_grad_enabled():   # create_graph: a gradient that is differentiated in turn
-            loss = _torch_loss_sum(logits, target, ctx.ignore_index)
-            return torch.autograd.grad(loss, logits, gout, create_graph=True)[0], None, None
+        if not _plain_backward(gout):
+            return _logits_gradient(logits, target, ctx.ignore_index, gout), None, None
         return _hip.load().cross_entropy_backward(logits, target, ctx.ignore_index, stats, gout), None, None
 
 
@@ -129,19 +153,21 @@ class _HeadLoss(torch.autograd.Function):
     def backward(ctx, gout):
         (h, targets), weight = ctx.saved_tensors, ctx.weight
         wanted = ctx.needs_input_grad[:2]
+        parts = zip(torch.split(h, ctx.chunk), torch.split(targets, ctx.chunk))
         with torch.autocast(h.device.type, enabled=False):   # as the forward ran (_head_applies)
-            if torch.is_grad_enabled():   # create_graph: gradients that are differentiated in turn
-                total = sum(_torch_loss_sum(torch.mm(a, weight.t()), t, ctx.ignore_index)
-                            for a, t in zip(torch.split(h, ctx.chunk), torch.split(targets, ctx.chunk)))
-                inputs = [x for x, want in zip((h, weight), wanted) if want]
-                grads = iter(torch.autograd.grad(total, inputs, gout, create_graph=True))
-                return (*(next(grads) if want else None for want in wanted), None, None, None)
+            if not _plain_backward(gout):
+                dh, dw = [], 0.0
+                for h_part, t_part in parts:
+                    grad = _logits_gradient(torch.mm(h_part, weight.t()), t_part, ctx.ignore_index, gout)
+                    if wanted[0]:
+                        dh.append(torch.mm(grad, weight))
+                    if wanted[1]:
+                        dw = dw + torch.mm(grad.t(), h_part)
+                return torch.cat(dh) if wanted[0] else None, dw if wanted[1] else None, None, None, None
             k = _hip.load()
             dh = torch.empty_like(h) if wanted[0] else None
             dw = None
-            parts = zip(torch.split(h, ctx.chunk), torch.split(targets, ctx.chunk),
-                        torch.split(h if dh is None else dh, ctx.chunk))
-            for h_part, t_part, dh_part in parts:
+            for (h_part, t_part), dh_part in zip(parts, torch.split(h if dh is None else dh, ctx.chunk)):
                 logits = torch.mm(h_part, weight.t())
                 stats = k.cross_entropy(logits, t_part, ctx.ignore_index)[1]
                 grad = k.cross_entropy_backward(logits, t_part, ctx.ignore_index, stats, gout, out=logits)
@@ -167,7 +193,7 @@ def _slice_loss_sum(h: torch.Tensor, target: torch.Tensor, project: Callable[[to
     if not _kernels_apply(logits, target, observed):
         return _torch_loss_sum(logits, target, ignore_index)
     if torch.is_grad_enabled() and logits.requires_grad:
-        return _SliceLoss.apply(logits, target, ignore_index)
+        return _SliceLoss.apply(logits, target, ignore_index)[0]
     return _hip.load().cross_entropy(logits, target, ignore_index)[0]
 
 

@@ -236,3 +236,46 @@ def test_which_products_are_split(monkeypatch):
     assert not try_(8, 64, 8192) and not try_(8, 66, 1 << 14) and not try_(8, 64, 20004)
     assert not try_(8, 64, 1 << 14, torch.float32) and not try_(8, 64, 1 << 14, offset=4)
     assert not try_(2056, 2048, 1 << 14)
+
+
+@pytest.mark.parametrize("bias", [False, True])
+def test_backward_passes_of_other_kinds(bias, monkeypatch):
+    """Batched gradients, a pass under autocast, a default device, a step between the forward and the backward
+    pass: on the kernels where they apply, the torch operations' results everywhere."""
+    hidden, head, labels = _problem(torch.float32, vocab=1 << 14)
+    if bias:
+        head.bias = torch.nn.Parameter(torch.zeros(1 << 14, device="cuda"))
+    seeds = torch.tensor([1.0, -0.3], device="cuda")
+
+    def results(kernels):
+        inputs = [hidden, *head.parameters()]
+        opt = ab.AdamBridge(head.parameters(), lr=1e-2)
+        start = head.weight.detach().clone()
+        out = list(torch.autograd.grad(ab.causal_lm_loss(hidden, head, labels, chunk_tokens=32), inputs, seeds,
+                                       is_grads_batched=True))
+        loss = ab.causal_lm_loss(hidden, head, labels, chunk_tokens=32)
+        with torch.autocast("cuda", dtype=torch.bfloat16, enabled=not bias and kernels):   # torch's products take BF16 there
+            out += torch.autograd.grad(loss, inputs)
+        torch.set_default_device("cuda")
+        try:
+            out += torch.autograd.grad(ab.causal_lm_loss(hidden, head, labels, chunk_tokens=32), inputs)
+        finally:
+            torch.set_default_device(None)
+        loss = ab.causal_lm_loss(hidden, head, labels, chunk_tokens=32)
+        for p in head.parameters():   # the same update on both sides
+            p.grad = torch.randn(p.shape, generator=torch.Generator("cuda").manual_seed(5), device="cuda")
+        opt.step()
+        out += torch.autograd.grad(loss, inputs)
+        with torch.no_grad():
+            head.weight.copy_(start)
+            head.weight.grad = None
+            if bias:
+                head.bias.zero_()
+                head.bias.grad = None
+        return out
+
+    got = results(True)
+    monkeypatch.setattr(losses, "_head_applies", lambda *a: False)
+    monkeypatch.setattr(losses, "_kernels_apply", lambda *a: False)
+    for i, (a, b) in enumerate(zip(got, results(False), strict=True)):
+        assert a.dtype == b.dtype == torch.float32 and (a - b).norm() <= 1e-5 * b.norm(), i   # as in the tests above

@@ -193,3 +193,45 @@ def test_a_default_device_does_not_keep_the_kernels_away(kernels, bias):
         assert not kernels.calls
     finally:
         torch.set_default_device(None)
+
+
+@pytest.mark.parametrize("head_kind", ["bias", "linear", "frozen"])
+def test_batched_gradients(kernels, head_kind):
+    """is_grads_batched: the backward pass runs under vmap, its incoming gradient a batch."""
+    hidden, head, labels = _problem(bias=head_kind == "bias")
+    hidden.requires_grad_(head_kind != "frozen")
+    inputs = [x for x in (hidden, *head.parameters()) if x.requires_grad]
+    seeds = torch.tensor([0.0, 1.0, -0.3])
+    want = torch.autograd.grad(_whole(hidden, head, labels), inputs)
+    got = torch.autograd.grad(_loss(hidden, head, labels), inputs, seeds, is_grads_batched=True)
+    for g, w in zip(got, want, strict=True):
+        assert _close(list(g[1:]), [seeds[1] * w, seeds[2] * w]) and not g[0].any()
+    loss = _loss(hidden, head, labels)
+    for g, b in zip(got, torch.func.vmap(lambda seed: torch.autograd.grad(loss, inputs, seed))(seeds), strict=True):
+        assert torch.allclose(g, b, rtol=1e-5, atol=1e-7)
+
+
+@pytest.mark.parametrize("head_kind", ["bias", "linear"])
+def test_vectorized_jacobians_and_second_derivatives(kernels, head_kind):
+    hidden, head, labels = _problem(bias=head_kind == "bias")
+    jacobian = torch.autograd.functional.jacobian(lambda h: _loss(h, head, labels), hidden.detach(), vectorize=True)
+    assert _close([jacobian], torch.autograd.grad(_whole(hidden, head, labels), hidden))
+    inputs = [hidden, head.weight]
+
+    def second(loss):
+        first = torch.autograd.grad(loss, inputs, torch.tensor(0.7), create_graph=True)
+        return torch.autograd.grad(sum(g.square().sum() for g in first), inputs)
+
+    assert _close(second(_loss(hidden, head, labels)), second(_whole(hidden, head, labels)), 1e-4)
+
+
+def test_operations_watched_in_the_backward_pass_are_torchs(kernels):
+    from torch.utils.flop_counter import FlopCounterMode
+    hidden, head, labels = _problem(torch.bfloat16, vocab=1 << 14)
+    inputs = [hidden, head.weight]
+    want = torch.autograd.grad(_whole(hidden, head, labels), inputs)
+    loss = _loss(hidden, head, labels)
+    with FlopCounterMode(display=False) as count:
+        got = torch.autograd.grad(loss, inputs)
+    assert count.get_total_flops() == 3 * 2 * 24 * 8 * (1 << 14) and "matmul" not in kernels.calls
+    assert _close(got, want, 2.0 ** -7)   # the logits' gradient and the result rounded to BF16
