@@ -200,7 +200,9 @@ __global__ __launch_bounds__(kFinishThreads) void k_ce_finish(const void* logits
 }
 
 // grad = (exp(x - m) / s - [k == target]) * gout for a row's values, 0 * that for an ignored row (a NaN
-// row stays NaN there, as in the composition this replaces).  Workgroups as in k_ce_partial.
+// row stays NaN there, as in the composition this replaces), NaN for a row whose target lies outside
+// [0, vocab), as its loss is: an update must not follow a gradient that no loss has.  Workgroups as in
+// k_ce_partial.
 template <int DT>
 __global__ __launch_bounds__(kCeThreads) void k_ce_backward(const void* logits, const int64_t* target, int64_t vocab,
                                                             int64_t ignore, int32_t splits, const float* stats,
@@ -214,7 +216,7 @@ __global__ __launch_bounds__(kCeThreads) void k_ce_backward(const void* logits, 
     uint8_t* out = static_cast<uint8_t*>(grad) + row * vocab * size;
     const int64_t t = target[row];
     const float m = stats[2 * row], inv = stats[2 * row + 1];
-    const float g = t == ignore ? 0.0f : gout[0];
+    const float g = t == ignore ? 0.0f : t < 0 || t >= vocab ? __builtin_nanf("") : gout[0];
     const float f = inv * g;
     const int64_t head = head_of<DT>(base, vocab);
     const int64_t nvec = (vocab - head) / K;

@@ -84,8 +84,9 @@ def _logits_gradient(logits: torch.Tensor, target: torch.Tensor, ignore_index: i
     """What ``cross_entropy_backward`` computes, in torch operations: differentiable, and for a ``gout`` that is
     a batch (vmap)."""
     p = logits.float().softmax(1)
-    seed = torch.where(target == ignore_index, 0.0, gout)[:, None]   # an ignored row: 0 times what it holds
     at = target.clamp(0, logits.shape[1] - 1)[:, None]
+    seed = torch.where(at[:, 0] == target, gout, torch.nan)                 # no such class: no gradient
+    seed = torch.where(target == ignore_index, 0.0, seed)[:, None]   # an ignored row: 0 times what it holds
     return (p.scatter_add(1, at, p.new_full((), -1.0).expand_as(at)) * seed).to(logits.dtype)
 
 

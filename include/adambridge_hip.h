@@ -490,8 +490,8 @@ ADAMBRIDGE_API int adambridge_matmul(const void* a, const void* b, void* c, int6
  * exponentials); work holds adambridge_cross_entropy_work(rows, vocab) bytes of scratch, 8-byte
  * aligned.  adambridge_cross_entropy_backward writes (softmax - one_hot(target)) * gout[0] to grad, in
  * the logits' type; grad may be logits.  All of it is computed in FP32; sums are taken in a fixed order.  A target
- * outside [0, vocab) other than ignore_index makes the loss NaN (nothing is read for it).  Returns 0,
- * ADAMBRIDGE_EBADN (rows outside 1 .. 2^23, vocab < 1), _EMVDTYPE, _ENULL, _EALIGN (grad at another offset
+ * outside [0, vocab) other than ignore_index makes the loss and its row's gradient NaN (nothing is read for it).
+ * Returns 0, ADAMBRIDGE_EBADN (rows outside 1 .. 2^23, vocab < 1), _EMVDTYPE, _ENULL, _EALIGN (grad at another offset
  * from a 16-byte boundary than logits) or _EHIP; adambridge_cross_entropy_work the bytes, or
  * ADAMBRIDGE_EBADN. */
 ADAMBRIDGE_API int64_t adambridge_cross_entropy_work(int64_t rows, int64_t vocab);

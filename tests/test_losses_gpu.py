@@ -279,3 +279,18 @@ def test_backward_passes_of_other_kinds(bias, monkeypatch):
     monkeypatch.setattr(losses, "_kernels_apply", lambda *a: False)
     for i, (a, b) in enumerate(zip(got, results(False), strict=True)):
         assert a.dtype == b.dtype == torch.float32 and (a - b).norm() <= 1e-5 * b.norm(), i   # as in the tests above
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("vocab", [7, 300, 20001])   # the row in values, in vectors with a tail, over several workgroups
+def test_a_target_outside_the_vocabulary_has_no_gradient(vocab, dtype):
+    """NaN over its whole row, as the loss is, and in no other."""
+    logits, target = _case(6, vocab, dtype)
+    target[1], target[2], target[4] = vocab, -1, vocab + 5
+    k = _hip.load()
+    loss, stats = k.cross_entropy(logits, target, IGNORE)
+    for gout in (torch.ones((), device="cuda"), torch.zeros((), device="cuda")):
+        grad = k.cross_entropy_backward(logits, target, IGNORE, stats, gout)
+        same = losses._logits_gradient(logits, target, IGNORE, gout)
+        for g in (grad, same):
+            assert loss.isnan() and g[[1, 2, 4]].isnan().all() and not g[[0, 3, 5]].isnan().any()

@@ -235,3 +235,14 @@ def test_operations_watched_in_the_backward_pass_are_torchs(kernels):
         got = torch.autograd.grad(loss, inputs)
     assert count.get_total_flops() == 3 * 2 * 24 * 8 * (1 << 14) and "matmul" not in kernels.calls
     assert _close(got, want, 2.0 ** -7)   # the logits' gradient and the result rounded to BF16
+
+
+def test_a_target_outside_the_vocabulary_has_no_gradient_in_torch_operations_either():
+    logits = torch.randn(5, 9, generator=torch.Generator().manual_seed(2), requires_grad=True)
+    target = torch.tensor([3, 9, IGNORE, -1, 8])
+    grad = losses._logits_gradient(logits, target, IGNORE, torch.tensor(0.0))
+    assert grad[[1, 3]].isnan().all() and not grad[[0, 2, 4]].any()
+    good = [0, 2, 4]
+    loss = F.cross_entropy(logits[good], target[good], ignore_index=IGNORE, reduction="sum")
+    want = torch.autograd.grad(loss, logits)[0][good]
+    assert torch.allclose(losses._logits_gradient(logits, target, IGNORE, torch.tensor(1.0))[good], want, atol=1e-6)
