@@ -17,6 +17,8 @@
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <cstdint>
+#include <exception>
+#include <new>
 #include <vector>
 
 #include "../../include/adambridge_hip.h"
@@ -82,7 +84,7 @@ struct Found {
 // writes the segments' addresses to `array` (a ctypes array of pointers).  False, with nothing
 // changed, if any slot needs the general path.  group_address(group) gives the address of a
 // parameter group's adambridge_group, refreshed from its dict; it is called once per group.
-PyObject* describe(PyObject*, PyObject* const* args, Py_ssize_t nargs)
+PyObject* describe_slots(PyObject* const* args, Py_ssize_t nargs)
 {
     if (nargs != 7 || !PyList_CheckExact(args[0]) || !PyList_CheckExact(args[1])) {
         PyErr_SetString(PyExc_TypeError, "describe(slots, grads, array, device, algorithm, delay, group_address)");
@@ -171,8 +173,22 @@ PyObject* describe(PyObject*, PyObject* const* args, Py_ssize_t nargs)
     Py_RETURN_TRUE;
 }
 
+// C++ exceptions end here.  Torch's come from the checks (a tensor without memory of its own), before
+// anything was written: the general path meets the same tensor and raises in Python.
+PyObject* describe(PyObject*, PyObject* const* args, Py_ssize_t nargs)
+{
+    try {
+        return describe_slots(args, nargs);
+    } catch (const std::bad_alloc&) {
+        return PyErr_NoMemory();
+    } catch (const std::exception&) {
+        PyErr_Clear();
+        Py_RETURN_FALSE;
+    }
+}
+
 // pending(slots, include_small) -> (slots, grads): those not updated in this step that have a gradient.
-PyObject* pending(PyObject*, PyObject* const* args, Py_ssize_t nargs)
+PyObject* pending_slots(PyObject* const* args, Py_ssize_t nargs)
 {
     if (nargs != 2 || !PyList_CheckExact(args[0])) {
         PyErr_SetString(PyExc_TypeError, "pending(slots, include_small)");
@@ -207,6 +223,18 @@ PyObject* pending(PyObject*, PyObject* const* args, Py_ssize_t nargs)
         if (PyList_Append(slots.o, slot) < 0 || PyList_Append(grads.o, grad.o) < 0) return nullptr;
     }
     return PyTuple_Pack(2, slots.o, grads.o);
+}
+
+PyObject* pending(PyObject*, PyObject* const* args, Py_ssize_t nargs)
+{
+    try {
+        return pending_slots(args, nargs);
+    } catch (const std::bad_alloc&) {
+        return PyErr_NoMemory();
+    } catch (const std::exception& e) {
+        PyErr_SetString(PyExc_RuntimeError, e.what());
+        return nullptr;
+    }
 }
 
 // mark(slots, submitted): sets the flag of each.
