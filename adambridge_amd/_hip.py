@@ -379,17 +379,29 @@ class HipKernels:
         into the arrays (adambridge_unpack_state).  The memory must stay alive until the stream has
         run it."""
         fn = self._lib.adambridge_pack_state if pack else self._lib.adambridge_unpack_state
+        rc = self._on(device, fn, ctypes.byref(state), ctypes.byref(arrays))
+        self._check(rc, "adambridge_pack_state" if pack else "adambridge_unpack_state")
+
+    def _on(self, device: torch.device, fn, *args) -> int:
+        """``fn(*args)`` with ``device`` current and its current stream the library's.  (Calls come one by one for
+        a model's states or a loss's slices: no context to enter where the device is current already.)"""
         current = torch._C._cuda_getDevice()
         index = current if device.index is None else device.index
         self._lib.adambridge_set_stream(torch._C._cuda_getCurrentRawStream(index))
-        if index == current:   # a model's states are moved one by one: no context to enter for each
-            rc = fn(ctypes.byref(state), ctypes.byref(arrays))
-        else:
-            with torch.cuda.device(index):
-                rc = fn(ctypes.byref(state), ctypes.byref(arrays))
-        self._check(rc, "adambridge_pack_state" if pack else "adambridge_unpack_state")
+        if index == current:
+            return fn(*args)
+        with torch.cuda.device(index):
+            return fn(*args)
 
     # -- cross-entropy ---------------------------------------------------------
+
+    @staticmethod
+    def _operand(name: str, t: torch.Tensor, dtypes: tuple, shape: tuple, device: torch.device) -> None:
+        """The kernels take addresses and sizes as they are given: raises ValueError unless ``t`` is what they
+        read or write there."""
+        if t.dtype not in dtypes or tuple(t.shape) != shape or not t.is_contiguous() or t.device != device:
+            raise ValueError(f"{name} must be contiguous, {shape} of {' or '.join(map(str, dtypes))} on {device}, got "
+                             f"{tuple(t.shape)} of {t.dtype} on {t.device} with strides {t.stride()}")
 
     def cross_entropy(self, logits: torch.Tensor, target: torch.Tensor, ignore_index: int
                       ) -> tuple[torch.Tensor, torch.Tensor]:
@@ -397,17 +409,16 @@ class HipKernels:
         classes, on the current stream (adambridge_cross_entropy): the FP32 sum and the per-row
         statistics its gradient takes."""
         rows, vocab = logits.shape
+        self._operand("logits", logits, (torch.float32, torch.bfloat16), (rows, vocab), logits.device)
+        self._operand("target", target, (torch.int64,), (rows,), logits.device)
         nbytes = self._lib.adambridge_cross_entropy_work(rows, vocab)
         if nbytes < 0:
             self._check(nbytes, "adambridge_cross_entropy_work")
         work = torch.empty(nbytes // 4, dtype=torch.float32, device=logits.device)
         stats = torch.empty(rows, 2, dtype=torch.float32, device=logits.device)
         loss = torch.empty((), dtype=torch.float32, device=logits.device)
-        with torch.cuda.device(logits.device):
-            self._lib.adambridge_set_stream(torch.cuda.current_stream(logits.device).cuda_stream)
-            rc = self._lib.adambridge_cross_entropy(logits.data_ptr(), _DTYPE_CODES[logits.dtype], target.data_ptr(), rows,
-                                                    vocab, ignore_index, work.data_ptr(), stats.data_ptr(),
-                                                    loss.data_ptr())
+        rc = self._on(logits.device, self._lib.adambridge_cross_entropy, logits.data_ptr(), _DTYPE_CODES[logits.dtype],
+                      target.data_ptr(), rows, vocab, ignore_index, work.data_ptr(), stats.data_ptr(), loss.data_ptr())
         self._check(rc, "adambridge_cross_entropy")
         return loss, stats
 
@@ -419,24 +430,28 @@ class HipKernels:
         or ``out``, which may be the logits themselves."""
         rows, vocab = logits.shape
         grad = torch.empty_like(logits) if out is None else out
-        with torch.cuda.device(logits.device):
-            self._lib.adambridge_set_stream(torch.cuda.current_stream(logits.device).cuda_stream)
-            rc = self._lib.adambridge_cross_entropy_backward(
-                logits.data_ptr(), _DTYPE_CODES[logits.dtype], target.data_ptr(), rows, vocab, ignore_index,
-                stats.data_ptr(), gout.data_ptr(), grad.data_ptr())
+        self._operand("logits", logits, (torch.float32, torch.bfloat16), (rows, vocab), logits.device)
+        self._operand("target", target, (torch.int64,), (rows,), logits.device)
+        self._operand("stats", stats, (torch.float32,), (rows, 2), logits.device)
+        self._operand("gout", gout, (torch.float32,), (), logits.device)
+        self._operand("out", grad, (logits.dtype,), (rows, vocab), logits.device)
+        rc = self._on(logits.device, self._lib.adambridge_cross_entropy_backward, logits.data_ptr(),
+                      _DTYPE_CODES[logits.dtype], target.data_ptr(), rows, vocab, ignore_index, stats.data_ptr(),
+                      gout.data_ptr(), grad.data_ptr())
         self._check(rc, "adambridge_cross_entropy_backward")
         return grad
 
     def matmul(self, a: torch.Tensor, b: torch.Tensor, out: torch.Tensor) -> None:
         """``out`` = ``a @ b`` for contiguous bfloat16 matrices on the current stream (adambridge_matmul)."""
         (m, k), n = a.shape, b.shape[1]
+        for name, t, shape in (("a", a, (m, k)), ("b", b, (k, n)), ("out", out, (m, n))):
+            self._operand(name, t, (torch.bfloat16,), shape, a.device)
         nbytes = self._lib.adambridge_matmul_work(m, n, k)
         if nbytes < 0:
             self._check(nbytes, "adambridge_matmul_work")
         work = torch.empty(nbytes // 4, dtype=torch.float32, device=a.device)
-        with torch.cuda.device(a.device):
-            self._lib.adambridge_set_stream(torch.cuda.current_stream(a.device).cuda_stream)
-            rc = self._lib.adambridge_matmul(a.data_ptr(), b.data_ptr(), out.data_ptr(), m, n, k, work.data_ptr())
+        rc = self._on(a.device, self._lib.adambridge_matmul, a.data_ptr(), b.data_ptr(), out.data_ptr(), m, n, k,
+                      work.data_ptr())
         self._check(rc, "adambridge_matmul")
 
     def fused_adamw(self, master: torch.Tensor, grad: torch.Tensor, m: torch.Tensor, v: torch.Tensor,

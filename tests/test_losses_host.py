@@ -246,3 +246,37 @@ def test_a_target_outside_the_vocabulary_has_no_gradient_in_torch_operations_eit
     loss = F.cross_entropy(logits[good], target[good], ignore_index=IGNORE, reduction="sum")
     want = torch.autograd.grad(loss, logits)[0][good]
     assert torch.allclose(losses._logits_gradient(logits, target, IGNORE, torch.tensor(1.0))[good], want, atol=1e-6)
+
+
+class _Library:
+    """The loaded library where no call may reach it."""
+
+    def __getattr__(self, name):
+        raise AssertionError(f"{name} was called")
+
+
+def test_operands_the_kernels_cannot_take_are_refused():
+    """Types, shapes, strides and devices are checked before an address is passed on."""
+    k = object.__new__(_hip.HipKernels)
+    k._lib = _Library()
+    bf16 = dict(dtype=torch.bfloat16)
+
+    a, b, out = torch.zeros(4, 16, **bf16), torch.zeros(16, 8, **bf16), torch.zeros(4, 8, **bf16)
+    for wrong in ((a.float(), b, out), (a, b.float(), out), (a, b, out.float()), (a, b, out[:3]), (a, b[:8], out),
+                  (a, b, torch.zeros(8, 4, **bf16).t()), (a.t().contiguous().t(), b, out), (a, b, out.to("meta"))):
+        with pytest.raises(ValueError, match="must be contiguous"):
+            k.matmul(*wrong)
+
+    x, t = torch.zeros(4, 9), torch.zeros(4, dtype=torch.int64)
+    for wrong in ((x.half(), t), (x.t().contiguous().t(), t), (x, t.int()), (x, t[:3]), (x, t.to("meta")),
+                  (x, torch.zeros(8, dtype=torch.int64)[::2])):
+        with pytest.raises(ValueError, match="must be contiguous"):
+            k.cross_entropy(*wrong, IGNORE)
+
+    stats, gout = torch.zeros(4, 2), torch.zeros(())
+    for wrong in ((x, t, stats[:3], gout, None), (x, t, stats.double(), gout, None), (x, t, stats, gout.double(), None),
+                  (x, t, stats, gout[None], None), (x, t, stats, gout, x.bfloat16()), (x, t, stats, gout, x[:, :8]),
+                  (x, t.int(), stats, gout, None), (x.half(), t, stats, gout, None), (x, t, stats, gout.to("meta"), None)):
+        logits, target, s, g, o = wrong
+        with pytest.raises(ValueError, match="must be contiguous"):
+            k.cross_entropy_backward(logits, target, IGNORE, s, g, o)
