@@ -91,9 +91,28 @@ def _logits_gradient(logits: torch.Tensor, target: torch.Tensor, ignore_index: i
 
 
 class _SliceLoss(torch.autograd.Function):
-    """Summed cross-entropy by the library's kernels, and the two floats per row that are kept for the
-    backward pass beside the logits themselves.  (Forward and context apart: a checkpointed slice may be
-    computed again while a batched backward pass runs under vmap, on tensors that are not batched.)"""
+    """Summed cross-entropy by the library's kernels.  What is kept for the backward pass is the logits
+    themselves and two floats per row."""
+
+    @staticmethod
+    def forward(ctx, logits, target, ignore_index):
+        loss, stats = _hip.load().cross_entropy(logits, target, ignore_index)
+        ctx.save_for_backward(logits, target, stats)
+        ctx.ignore_index = ignore_index
+        return loss
+
+    @staticmethod
+    def backward(ctx, gout, *_):
+        logits, target, stats = ctx.saved_tensors
+        if not _plain_backward(gout):
+            return _logits_gradient(logits, target, ctx.ignore_index, gout), None, None
+        return _hip.load().cross_entropy_backward(logits, target, ctx.ignore_index, stats, gout), None, None
+
+
+class _SliceLossInTransform(_SliceLoss):
+    """The same in the form that may run while a function transform is active, on tensors that are no part of
+    it: a checkpointed slice computed again in a backward pass under vmap.  (A call of this form costs
+    the host 30 us more.)"""
 
     @staticmethod
     def forward(logits, target, ignore_index):
@@ -109,13 +128,6 @@ class _SliceLoss(torch.autograd.Function):
     @staticmethod
     def vmap(info, in_dims, logits, target, ignore_index):
         raise NotImplementedError("batched logits take the torch operations (_kernels_apply)")
-
-    @staticmethod
-    def backward(ctx, gout, _):
-        logits, target, stats = ctx.saved_tensors
-        if not _plain_backward(gout):
-            return _logits_gradient(logits, target, ctx.ignore_index, gout), None, None
-        return _hip.load().cross_entropy_backward(logits, target, ctx.ignore_index, stats, gout), None, None
 
 
 def _matmul_into(out: torch.Tensor, a: torch.Tensor, b: torch.Tensor) -> None:
@@ -194,7 +206,9 @@ def _slice_loss_sum(h: torch.Tensor, target: torch.Tensor, project: Callable[[to
     if not _kernels_apply(logits, target, observed):
         return _torch_loss_sum(logits, target, ignore_index)
     if torch.is_grad_enabled() and logits.requires_grad:
-        return _SliceLoss.apply(logits, target, ignore_index)[0]
+        if torch._C._are_functorch_transforms_active():
+            return _SliceLossInTransform.apply(logits, target, ignore_index)[0]
+        return _SliceLoss.apply(logits, target, ignore_index)
     return _hip.load().cross_entropy(logits, target, ignore_index)[0]
 
 
