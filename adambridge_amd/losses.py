@@ -30,6 +30,23 @@ __all__ = ["causal_lm_loss"]
 _MAX_ROWS = 1 << 23   # adambridge_cross_entropy's
 
 
+# The kernels give each row a workgroup, which is mostly idle for a short one: from some number of rows on, torch's
+# softmax, several short rows a workgroup, is faster.  (Rows up to which the kernels are taken whatever
+# the vocabulary, and the vocabulary from which they are taken whatever the rows.)  Measured on MI355X, us,
+# kernels / torch operations.  A slice's loss alone, BF16: 2^14 rows of 2 to 2048 values 97-122 / 98-165;
+# 2^15 x 256 124 / 105; 2^16 x 2 153 / 95, x 256 200 / 153, x 512 216 / 226; 2^20 x 8 1893 / 770, x 512 3501 /
+# 3447; FP32: 2^15 x 512 144 / 124, x 1000 185 / 186, 2^17 x 512 496 / 450, x 1000 671 / 730.  A training pass of
+# a bare Linear head, with its other savings, BF16: 2^16 x 2 593 / 616, x 128 609 / 753; 2^17 x 8 856 / 758, x 128
+# 1058 / 891, x 256 1136 / 1218; 2^18 x 256 1979 / 2335; FP32: 2^16 x 2 544 / 726; 2^17 x 256 1200 / 1186, 2^18 x 512
+# 2930 / 3215.
+_SLICE_RULE = (1 << 14, {torch.bfloat16: 512, torch.float32: 1000})
+_HEAD_RULE = (1 << 16, {torch.bfloat16: 256, torch.float32: 512})
+
+
+def _long_enough(rule: tuple, rows: int, vocab: int, dtype: torch.dtype) -> bool:
+    return rows <= rule[0] or vocab >= rule[1][dtype]
+
+
 def _observed() -> bool:
     """Whether something needs the torch operations themselves: a trace or compilation, a function
     transform (vmap, functorch grad), forward-mode derivatives, a mode that observes operations (a
@@ -53,10 +70,11 @@ def _ordinary(values: torch.Tensor, target: torch.Tensor) -> bool:
 def _kernels_apply(logits: torch.Tensor, target: torch.Tensor, observed: bool | None = None) -> bool:
     """Whether the library's cross-entropy takes this slice (``observed``: :func:`_observed`, if asked before)."""
     return (not (_observed() if observed is None else observed) and type(logits) is torch.Tensor and _ordinary(logits, target)
+            and _long_enough(_SLICE_RULE, *logits.shape, logits.dtype)
             and logits.data_ptr() % 16 == 0)   # so that the gradient, a new tensor, shares its alignment
 
 
-def _head_applies(head, h: torch.Tensor, targets: torch.Tensor) -> bool:
+def _head_applies(head, h: torch.Tensor, targets: torch.Tensor, chunk: int = 1) -> bool:
     """Whether ``head(h)`` is exactly ``h @ head.weight.T`` on plain tensors, so that :class:`_HeadLoss` may
     take the products itself: a torch.nn.Linear without a bias, with nothing hooked, replaced or cast
     around its call."""
@@ -70,7 +88,8 @@ def _head_applies(head, h: torch.Tensor, targets: torch.Tensor) -> bool:
     w = head.weight
     return (type(h) in (torch.Tensor, torch.nn.Parameter) and type(w) in (torch.Tensor, torch.nn.Parameter)
             and _ordinary(h, targets) and w.device == h.device and w.dtype == h.dtype and w.dim() == 2
-            and w.is_contiguous() and not w.is_neg() and w.shape[1] == h.shape[1] and w.shape[0] > 0)
+            and w.is_contiguous() and not w.is_neg() and w.shape[1] == h.shape[1] and w.shape[0] > 0
+            and _long_enough(_HEAD_RULE, min(chunk, h.shape[0]), w.shape[0], w.dtype))
 
 
 def _plain_backward(gout: torch.Tensor) -> bool:
@@ -239,7 +258,7 @@ def causal_lm_loss(hidden_states: torch.Tensor, lm_head: Callable[[torch.Tensor]
     targets = targets.reshape(-1).to(h.device)
     n_scored = (targets != ignore_index).sum()
     recompute = torch.is_grad_enabled() and h.requires_grad
-    if recompute and _head_applies(lm_head, h, targets):
+    if recompute and _head_applies(lm_head, h, targets, chunk_tokens):
         return _HeadLoss.apply(h, lm_head.weight, targets, ignore_index, chunk_tokens) / n_scored.clamp(min=1)
     observed = _observed()
     total = h.new_zeros((), dtype=torch.float32)

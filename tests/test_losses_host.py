@@ -280,3 +280,31 @@ def test_operands_the_kernels_cannot_take_are_refused():
         logits, target, s, g, o = wrong
         with pytest.raises(ValueError, match="must be contiguous"):
             k.cross_entropy_backward(logits, target, IGNORE, s, g, o)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_many_short_rows_take_torch_operations(kernels, dtype):
+    """Both sides of each line of the two rules: a slice's own kernels, and a bare Linear head's."""
+    def slice_taken(rows, vocab):
+        return losses._kernels_apply(torch.empty(rows, vocab, dtype=dtype), torch.empty(rows, dtype=torch.int64))
+
+    def head_taken(rows, vocab, chunk):
+        head = torch.nn.Linear(2, vocab, bias=False, dtype=dtype)
+        return losses._head_applies(head, torch.empty(rows, 2, dtype=dtype), torch.empty(rows, dtype=torch.int64), chunk)
+
+    few, line = losses._SLICE_RULE[0], losses._SLICE_RULE[1][dtype]
+    assert slice_taken(few, 1) and slice_taken(few, line) and slice_taken(few + 1, line)
+    assert not slice_taken(few + 1, line - 1) and not slice_taken(4 * few, 1)
+    few, line = losses._HEAD_RULE[0], losses._HEAD_RULE[1][dtype]
+    assert head_taken(few, 2, 2 * few) and head_taken(few + 1, line, 2 * few) and head_taken(4 * few, 2, few)
+    assert not head_taken(few + 1, line - 1, 2 * few)
+    hidden = torch.randn(1, few + 3, 2).to(dtype).requires_grad_()
+    head = torch.nn.Linear(2, 3, bias=False, dtype=dtype)
+    labels = torch.randint(0, 3, (1, few + 3))
+    for chunk, calls in ((few, True), (few + 3, False)):
+        kernels.calls.clear()
+        loss = ab.causal_lm_loss(hidden, head, labels, chunk_tokens=chunk)
+        assert bool(kernels.calls) == calls
+        got = torch.autograd.grad(loss, [hidden, head.weight])
+        tol = 1e-4 if dtype == torch.float32 else 2.0 ** -6   # FP32 sums of 65539 rows; BF16 logits and gradients
+        assert _close(got, torch.autograd.grad(_whole(hidden, head, labels), [hidden, head.weight]), tol)
