@@ -17,9 +17,9 @@
 // Measured on MI355X, us, the library's product beside it: 1024 x 896 over 151936 terms 346 (805
 // TFLOP/s) against 619; 333 x 896 196 / 451; 1024 x 4096 1346 / 1793; over 50264 terms 1024 x 2048 283 /
 // 484.  512 places are best (256: 508, 1024: 440); fragments read one step ahead, a raised wave priority
-// and the other order of tiles changed nothing (345-354).  The caller's rule (losses.py): 2^14 terms or
-// more and at most 2^22 results; beyond, the library is as fast or faster (4096 x 2048: 2635 / 1865, over 8192
-// terms 1024 x 896 39 / 44).
+// and the other order of tiles changed nothing (345-354).  The caller's rule (losses.py: _matmul_into): 2^14
+// terms or more, at most 4096 rows and 2^22 results (below 2^15 terms 2^21); beyond, the library is as fast
+// or faster (4096 x 2048: 2635 / 1865, 8192 x 512: 1460 / 1354, over 8192 terms 1024 x 896 39 / 44).
 
 #include <hip/hip_runtime.h>
 

@@ -308,3 +308,20 @@ def test_many_short_rows_take_torch_operations(kernels, dtype):
         got = torch.autograd.grad(loss, [hidden, head.weight])
         tol = 1e-4 if dtype == torch.float32 else 2.0 ** -6   # FP32 sums of 65539 rows; BF16 logits and gradients
         assert _close(got, torch.autograd.grad(_whole(hidden, head, labels), [hidden, head.weight]), tol)
+
+
+def test_which_products_are_worth_splitting(kernels):
+    def split(m, n, k):
+        kernels.calls.clear()
+        a, b, out = (torch.zeros(1, dtype=torch.bfloat16).expand(shape) for shape in ((m, k), (k, n), (m, n)))
+        kernels.matmul = lambda *x: kernels.calls.append("matmul")
+        try:
+            losses._matmul_into(out, a, b)
+        except RuntimeError:   # torch's product refuses an expanded result
+            pass
+        return bool(kernels.calls)
+
+    assert split(4096, 1024, 1 << 15) and split(1024, 4096, 1 << 15) and split(4096, 64, 1 << 15)
+    assert not split(4104, 64, 1 << 15) and not split(4096, 1028, 1 << 15)
+    assert split(2048, 1024, 1 << 14) and split(4096, 512, (1 << 15) - 8)
+    assert not split(2048, 1028, 1 << 14) and not split(4096, 516, (1 << 15) - 8) and not split(8, 64, (1 << 14) - 8)
