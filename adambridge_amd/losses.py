@@ -102,11 +102,12 @@ def _plain_backward(gout: torch.Tensor) -> bool:
 def _logits_gradient(logits: torch.Tensor, target: torch.Tensor, ignore_index: int, gout: torch.Tensor) -> torch.Tensor:
     """What ``cross_entropy_backward`` computes, in torch operations: differentiable, and for a ``gout`` that is
     a batch (vmap)."""
+    vocab = logits.shape[1]
     p = logits.float().softmax(1)
-    at = target.clamp(0, logits.shape[1] - 1)[:, None]
-    seed = torch.where(at[:, 0] == target, gout, torch.nan)                 # no such class: no gradient
-    seed = torch.where(target == ignore_index, 0.0, seed)[:, None]   # an ignored row: 0 times what it holds
-    return (p.scatter_add(1, at, p.new_full((), -1.0).expand_as(at)) * seed).to(logits.dtype)
+    hot = torch.arange(vocab, device=target.device) == target[:, None]
+    seed = torch.where((target < 0) | (target >= vocab), torch.nan, gout)   # no such class: no gradient
+    seed = torch.where(target == ignore_index, 0.0, seed)[:, None]          # an ignored row: 0 times what it holds
+    return ((p - hot.float()) * seed).to(logits.dtype)
 
 
 class _SliceLoss(torch.autograd.Function):

@@ -294,3 +294,22 @@ def test_a_target_outside_the_vocabulary_has_no_gradient(vocab, dtype):
         same = losses._logits_gradient(logits, target, IGNORE, gout)
         for g in (grad, same):
             assert loss.isnan() and g[[1, 2, 4]].isnan().all() and not g[[0, 3, 5]].isnan().any()
+
+
+@pytest.mark.parametrize("bias", [False, True])
+def test_second_derivatives_with_deterministic_algorithms(bias):
+    hidden, head, labels = _problem(torch.float32, vocab=61)
+    if bias:
+        head.bias = torch.nn.Parameter(torch.zeros(61, device="cuda"))
+    inputs = [hidden, head.weight]
+    results = []
+    for loss_of in (lambda: ab.causal_lm_loss(hidden, head, labels, chunk_tokens=32),
+                    lambda: F.cross_entropy(head(hidden[:, :-1]).flatten(0, 1), labels[:, 1:].flatten(), ignore_index=IGNORE)):
+        torch.use_deterministic_algorithms(True)
+        try:
+            first = torch.autograd.grad(loss_of(), inputs, create_graph=True)
+            results.append(torch.autograd.grad(sum(g.square().sum() for g in first), inputs))
+        finally:
+            torch.use_deterministic_algorithms(False)
+    for a, b in zip(*results):
+        assert (a - b).norm() <= 1e-4 * b.norm()   # as the second derivatives above
