@@ -408,8 +408,10 @@ def load_master_(store: MomentStore, saved: Any) -> None:
 
 
 def _borrowed(t: torch.Tensor, dtype: torch.dtype, device) -> bool:
-    """Whether a checkpoint's tensor can stand in a store as it is: its type, on ``device``, contiguous."""
-    return t.dtype == dtype and device is not None and t.device == torch.device(device) and t.is_contiguous()
+    """Whether a checkpoint's tensor can stand in a store as it is: its type, on ``device``, contiguous, and
+    its memory holding its values (no subclass, which may have none of its own; no pending negation)."""
+    return (type(t) in (torch.Tensor, torch.nn.Parameter) and t.dtype == dtype and device is not None
+            and t.device == torch.device(device) and t.is_contiguous() and not t.is_neg())
 
 
 def store_from_state_dict(state: Any, numel: int, role: str, device=None, borrow: bool = False) -> MomentStore:

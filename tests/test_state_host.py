@@ -3,7 +3,8 @@
 import pytest
 import torch
 
-from adambridge_amd.precision import BF16Store, FP8Store, FP32Store
+from adambridge_amd.optimizer import _CheckpointReader
+from adambridge_amd.precision import BF16Store, FP8Store, FP32Store, store_from_state_dict
 from adambridge_amd.state import AdamRecordState, F24RecordState, PairState
 
 
@@ -26,3 +27,29 @@ def test_arrays_of_another_size_are_refused_before_the_kernel_reads_them(cls, si
     assert not moved
     state._packed(torch.zeros(300), {"m": FP32Store(300), "v": BF16Store(300)})
     assert moved == [True, True]
+
+
+class _Sub(torch.Tensor):
+    """A subclass may hold its values elsewhere than in memory of its own."""
+
+
+@pytest.mark.parametrize("kind", ["negated", "subclass"])
+@pytest.mark.parametrize("form", ["fp32", "bf16", "fp8", "tensor"])
+def test_a_checkpoints_tensors_stand_in_a_store_only_as_memory_holding_their_values(form, kind):
+    """The packing kernel reads the memory at a store's address."""
+    x = torch.randn(300, generator=torch.Generator().manual_seed(1)).square()
+
+    def shown(t):   # the values of t, not in its memory
+        return torch._neg_view(t.neg()) if kind == "negated" else t.as_subclass(_Sub)
+
+    if form == "tensor":
+        got, want = _CheckpointReader.moment(shown(x), 300, "v", "bf16", x.device, borrow=True), FP32Store(300, init=x)
+    else:
+        want = {"fp32": FP32Store, "bf16": BF16Store}[form](300, init=x) if form != "fp8" else FP8Store(300, "v", init=x)
+        saved = want.state_dict()
+        name = "scale" if form == "fp8" else "data"
+        saved[name] = shown(saved[name])
+        got = store_from_state_dict(saved, 300, "v", device="cpu", borrow=True)
+    assert got.precision == want.precision
+    for a, b in zip(got.tensors, want.tensors, strict=True):
+        assert type(a) is torch.Tensor and not a.is_neg() and torch.equal(a.view(torch.uint8), b.view(torch.uint8))
