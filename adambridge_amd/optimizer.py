@@ -45,7 +45,7 @@ import torch._dynamo  # noqa: F401 -- imported here, not by the first torch.comp
 
 from . import _hip
 from .engine import ParamSlot, SmallGroup, StepStats, UpdateEngine
-from .precision import (FP32Store, _borrowed, _checked, bytes_per_param, canonical_master_precision, canonical_precision,
+from .precision import (FP32Store, _checked, _in_memory, bytes_per_param, canonical_master_precision, canonical_precision,
                         check_master_state, make_store, store_from_state_dict)
 
 __all__ = ["AdamBridge", "LionBridge", "OptiComputeAdamW", "AutoTuneConfig"]
@@ -301,9 +301,7 @@ class _CheckpointReader:
             values = saved.to(device, torch.float32)
             if borrow:
                 flat = values.detach().reshape(-1).contiguous()
-                if _borrowed(flat, torch.float32, device):
-                    return FP32Store.wrap(flat)
-                return FP32Store(numel, init=flat, device=device)
+                return FP32Store.wrap(flat) if _in_memory(flat) else FP32Store(numel, init=flat, device=device)
             return make_store(precision, numel, role, init=values, device=device)
         store = store_from_state_dict(saved, numel, role, device=device, borrow=borrow)
         if store.precision == precision or borrow:

@@ -407,11 +407,15 @@ def load_master_(store: MomentStore, saved: Any) -> None:
     store.write(0, store.numel, master_to_fp32(saved, store.numel, store.device))
 
 
+def _in_memory(t: torch.Tensor) -> bool:
+    """Whether a tensor's memory holds its values (no subclass, which may have none; no pending negation)."""
+    return (type(t) is torch.Tensor or type(t) is torch.nn.Parameter) and not t.is_neg()
+
+
 def _borrowed(t: torch.Tensor, dtype: torch.dtype, device) -> bool:
-    """Whether a checkpoint's tensor can stand in a store as it is: its type, on ``device``, contiguous, and
-    its memory holding its values (no subclass, which may have none of its own; no pending negation)."""
-    return (type(t) in (torch.Tensor, torch.nn.Parameter) and t.dtype == dtype and device is not None
-            and t.device == torch.device(device) and t.is_contiguous() and not t.is_neg())
+    """Whether a checkpoint's tensor can stand in a store as it is: its type, on ``device``, contiguous, in memory."""
+    return (t.dtype == dtype and device is not None and t.device == torch.device(device) and t.is_contiguous()
+            and _in_memory(t))
 
 
 def store_from_state_dict(state: Any, numel: int, role: str, device=None, borrow: bool = False) -> MomentStore:

@@ -362,9 +362,9 @@ class _Interleaved(ParamState):
         if master is not None:
             plane, keep = _master_source(master, self.numel, self.device)
             arrays.p, arrays.p_lo, arrays.p_dtype = plane.data, plane.lo, plane.dtype
-        for what, n in [("master weights", t.numel()) for t in keep] + [(f"moment {r}", s.numel) for r, s in moments.items()]:
+        for n in (*(t.numel() for t in keep), *(s.numel for s in moments.values())):
             if n != self.numel:   # the kernel reads as many as the state has
-                raise ValueError(f"{what}: {n} elements for a state of {self.numel}")
+                raise ValueError(f"master weights or a moment of {n} elements for a state of {self.numel}")
         by_format: dict[str, dict[str, MomentStore]] = {}
         for role in self.roles:
             if role in moments:
