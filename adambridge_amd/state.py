@@ -362,9 +362,13 @@ class _Interleaved(ParamState):
         if master is not None:
             plane, keep = _master_source(master, self.numel, self.device)
             arrays.p, arrays.p_lo, arrays.p_dtype = plane.data, plane.lo, plane.dtype
-        for n in (*(t.numel() for t in keep), *(s.numel for s in moments.values())):
-            if n != self.numel:   # the kernel reads as many as the state has
-                raise ValueError(f"master weights or a moment of {n} elements for a state of {self.numel}")
+        n = self.numel   # the kernel reads as many from each array
+        for t in keep:
+            if t.numel() != n:
+                raise ValueError(f"master weights of {t.numel()} elements for a state of {n}")
+        for store in moments.values():
+            if store.numel != n:
+                raise ValueError(f"a moment of {store.numel} elements for a state of {n}")
         by_format: dict[str, dict[str, MomentStore]] = {}
         for role in self.roles:
             if role in moments:
