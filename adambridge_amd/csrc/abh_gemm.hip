@@ -14,8 +14,8 @@
 // slot n / 4 + 32 (n mod 4), so that both the writes and the reads of 32 lanes are contiguous (the MFMA's
 // column i of tile t is column 4 i + t of the result).
 //
-// Measured on MI355X, us, the library's product beside it: 1024 x 896 over 151936 terms 346 (805
-// TFLOP/s) against 619; 333 x 896 196 / 451; 1024 x 4096 1346 / 1793; over 50264 terms 1024 x 2048 283 /
+// Measured on MI355X, us, the library's product beside it: 1024 x 896 over 151936 terms 346-359 (777-805
+// TFLOP/s; 318 within a training pass) against 619; 333 x 896 196 / 451; 1024 x 4096 1346 / 1793; over 50264 terms 1024 x 2048 283 /
 // 484.  512 places are best (256: 508, 1024: 440); fragments read one step ahead, a raised wave priority
 // and the other order of tiles changed nothing (345-354).  The caller's rule (losses.py: _matmul_into): 2^14
 // terms or more, at most 4096 rows and 2^22 results (below 2^15 terms 2^21); beyond, the library is as fast

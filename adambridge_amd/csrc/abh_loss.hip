@@ -5,12 +5,14 @@
 // logits once forward, and once more beside writing the gradient backward, so HBM bounds both.  In
 // place of the FP32 copy, the FP32 log-probabilities and their FP32 gradient that the composition
 // of library operations passes through memory (about 55 bytes per logit and step against 8 here),
-// the logits stay BF16 in memory and FP32 in registers, and what is kept between the passes is two
+// the logits stay BF16 in memory and FP32 in registers, and what the gradient needs beside them is two
 // floats per row: the row's maximum and the reciprocal of its sum of exponentials.  Measured on
-// MI355X at 1024 x 151936 BF16 logits: forward 59 us (5.3 TB/s of logits read), where the library's
-// FP32 copy and softmax took 141 + 464 us; backward 111 us (5.6 TB/s), where its zero-fill, softmax
-// gradient and BF16 copy took 57 + 520 + 156 us.  A training pass of 4 such slices with a 896-wide
-// head went from 15.17 to 8.02 ms, of which the head's matrix products are 6.8.
+// MI355X at 1024 x 151936 BF16 logits: forward 54-59 us (5.3-5.8 TB/s of logits read), where the library's
+// FP32 copy and softmax took 141 + 464 us; backward 109-111 us (5.6-5.7 TB/s; 92 where the logits have just
+// been read), where its zero-fill, softmax gradient and BF16 copy took 57 + 520 + 156 us.  A training
+// pass of 4 such slices with a 896-wide head, one box: torch operations 15.32 ms, these kernels in
+// checkpointed slices 8.13, and 6.63 in one function (losses.py: _HeadLoss), of which the head's
+// products are 5.4.
 //
 // Rows are spread over workgroups of 256 lanes, 16 bytes a lane and load.  A call of few rows
 // splits each row over several workgroups (ce_splits) so that all 256 CUs read; the partial maxima

@@ -224,8 +224,8 @@ def _torch_loss_sum(logits: torch.Tensor, target: torch.Tensor, ignore_index: in
 def _slice_loss_sum(h: torch.Tensor, target: torch.Tensor, project: Callable[[torch.Tensor], torch.Tensor],
                     ignore_index: int, observed: bool | None = None) -> torch.Tensor:
     """Summed cross-entropy of one slice.  A checkpointed slice is computed again in the backward pass, where
-    other modes may be active but the same tensors must be
-    saved: its caller passes what it found ``observed``."""
+    other modes may be active but the same tensors must be saved: its caller passes what it found
+    ``observed``."""
     logits = project(h)
     if not _kernels_apply(logits, target, observed):
         return _torch_loss_sum(logits, target, ignore_index)
