@@ -399,7 +399,7 @@ class HipKernels:
     def _operand(name: str, t: torch.Tensor, dtypes: tuple, shape: tuple, device: torch.device) -> None:
         """The kernels take addresses and sizes as they are given: raises ValueError unless ``t`` is what they
         read or write there."""
-        if t.dtype not in dtypes or tuple(t.shape) != shape or not t.is_contiguous() or t.device != device:
+        if t.dtype not in dtypes or t.shape != shape or not t.is_contiguous() or t.device != device:
             raise ValueError(f"{name} must be contiguous, {shape} of {' or '.join(map(str, dtypes))} on {device}, got "
                              f"{tuple(t.shape)} of {t.dtype} on {t.device} with strides {t.stride()}")
 
